@@ -158,8 +158,13 @@ hipEvent_t prof_event(mg_ctx *ctx) {
 mg_status mg_ws_reserve(mg_ctx *ctx, size_t bytes) {
   if (bytes <= ctx->ws_bytes) return MG_OK;
   if (ctx->ws) {
-    MG_HIP(hipStreamSynchronize(ctx->stream));
-    MG_HIP(hipFree(ctx->ws));
+    if (ctx->ws_captured) {
+      ctx->ws_old.push_back(ctx->ws);
+      ctx->ws_captured = false;
+    } else {
+      MG_HIP(hipStreamSynchronize(ctx->stream));
+      MG_HIP(hipFree(ctx->ws));
+    }
     ctx->ws = nullptr;
     ctx->ws_bytes = 0;
   }
@@ -167,6 +172,24 @@ mg_status mg_ws_reserve(mg_ctx *ctx, size_t bytes) {
   MG_HIP(hipMalloc(&ctx->ws, want));
   ctx->ws_bytes = want;
   return MG_OK;
+}
+
+bool mg_ws_optional(mg_ctx *ctx, size_t bytes) {
+  if (ctx->max_bytes >= 0 && (int64_t)bytes > ctx->max_bytes) return false;
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(ctx->stream, &st) != hipSuccess) {
+    (void)hipGetLastError();
+    st = hipStreamCaptureStatusActive;
+  }
+  if (st != hipStreamCaptureStatusNone) {
+    if (bytes > ctx->ws_bytes) return false;
+    ctx->ws_captured = true;
+    return true;
+  }
+  if (mg_ws_reserve(ctx, bytes) == MG_OK) return true;
+  g_last_error.clear();
+  (void)hipGetLastError();
+  return false;
 }
 
 mg_status mg_h2d_table(mg_ctx *ctx, void *dst_dev, const void *src_host, size_t bytes) {
@@ -244,6 +267,7 @@ mg_status mg_ctx_destroy(mg_ctx *ctx) {
   (void)hipSetDevice(ctx->device);
   if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
   if (ctx->ws) (void)hipFree(ctx->ws);
+  for (void *p : ctx->ws_old) (void)hipFree(p);
   for (int i = 0; i < MG_PIN_SLOTS; i++)
     if (ctx->pin_ev[i]) (void)hipEventDestroy(ctx->pin_ev[i]);
   for (const mg_prof_rec &r : ctx->prof_recs) {
@@ -380,6 +404,7 @@ mg_status mg_weight_release(mg_weight *w) {
   if (w->kind == MG_W_NBITS) mg_nbits_free(w);
   if (w->kind == MG_W_INT8) mg_int8_free(w);
   if (w->kind == MG_W_F32 && w->f32.b) (void)hipFree(w->f32.b);
+  if (w->kind == MG_W_F32 && w->f32.pair) (void)hipFree(w->f32.pair);
   delete w;
   return MG_OK;
 }
@@ -577,6 +602,24 @@ mg_status mg_weight_f32_create(mg_ctx *ctx, const float *b, int64_t rows, int64_
     (void)hipFree(w->f32.b);
     delete w;
     return mg_fail(MG_DEVICE_ERROR, "mg_weight_f32_create: upload failed");
+  }
+  // Its pair images; a weight without them (no memory left) runs on the fp32
+  // MFMA kernel.
+  if (bytes && N < MG_PAIR_MAX_N) {
+    const size_t pb = mg_pair_bytes(N, K);
+    if (hipMalloc(&w->f32.pair, pb) != hipSuccess) {
+      w->f32.pair = nullptr;
+      (void)hipGetLastError();
+    } else {
+      w->device_bytes += (int64_t)pb;
+      mg_status st = mg_pair_split(ctx, w->f32.b, N, K, w->f32.pair);
+      if (st == MG_OK && hipStreamSynchronize(ctx->stream) != hipSuccess)
+        st = mg_fail(MG_DEVICE_ERROR, "mg_weight_f32_create: upload failed");
+      if (st != MG_OK) {
+        (void)mg_weight_release(w);
+        return st;
+      }
+    }
   }
   *out = w;
   return MG_OK;
@@ -1341,12 +1384,19 @@ mg_status gemm_w(mg_ctx *ctx, const float *a, bool a_dev_ptr, int64_t rows, int6
   const size_t oa = a_dev_ptr ? 0 : s.take((size_t)(rows * K) * 4);
   const size_t oc = (c && !c_dev_ptr) ? s.take((size_t)nc * 4) : 0;
   const size_t oy = y_dev_ptr ? 0 : s.take((size_t)(rows * w->N) * 4);
-  q.kspl = mg_f32_ksplit(rows, K, 1);
+  // On pair images where the weight has them and the images of A (row chunks
+  // of at most 64 MiB) can be had; else on the fp32 MFMA kernel, which needs
+  // less workspace or none.
+  const int64_t chunk = std::max<int64_t>(64, ((64ll << 20) / (int64_t)mg_pair_bytes(64, K)) * 64);
+  const size_t pb = mg_align(mg_pair_bytes(std::min(rows, chunk), K));
+  const bool pair = w->f32.pair && mg_ws_optional(ctx, s.off + pb);
+  q.kspl = pair ? 1 : mg_f32_ksplit(rows, K, 1);
   // Partials of at most 64 MiB: wider weights run in column chunks.
   if (q.kspl > 1)
     q.part_cols = std::min<int64_t>(
         w->N, std::max<int64_t>(64, ((64ll << 20) / ((int64_t)q.kspl * rows * 4)) / 64 * 64));
-  const size_t op = q.kspl > 1 ? s.take((size_t)q.kspl * rows * q.part_cols * 4) : 0;
+  const size_t op = pair ? s.take(pb)
+                    : q.kspl > 1 ? s.take((size_t)q.kspl * rows * q.part_cols * 4) : 0;
   MG_TRY(mg_check_control(ctx, (int64_t)s.off));
   MG_TRY(mg_ws_reserve(ctx, s.off));
   char *base = static_cast<char *>(ctx->ws);
@@ -1366,7 +1416,18 @@ mg_status gemm_w(mg_ctx *ctx, const float *a, bool a_dev_ptr, int64_t rows, int6
     }
   }
   if (!y_dev_ptr) yd = reinterpret_cast<float *>(base + oy);
-  MG_TRY(mg_f32_run(ctx, q, ad, w->f32.b, yd));
+  if (pair) {
+    for (int64_t m0 = 0; m0 < rows; m0 += chunk) {
+      mg_f32_problem r = q;
+      r.M = std::min(chunk, rows - m0);
+      if (q.c) r.c = q.c + m0 * q.c_rs;
+      MG_TRY(mg_pair_split(ctx, ad + m0 * K, r.M, K, base + op));
+      MG_TRY(mg_pair_run(ctx, r, ad + m0 * K, base + op, w->f32.b, w->f32.pair,
+                         yd + m0 * w->N));
+    }
+  } else {
+    MG_TRY(mg_f32_run(ctx, q, ad, w->f32.b, yd));
+  }
   if (!y_dev_ptr) {
     MG_HIP(hipMemcpyAsync(y, yd, (size_t)(rows * w->N) * 4, hipMemcpyDeviceToHost, ctx->stream));
     MG_HIP(hipStreamSynchronize(ctx->stream));

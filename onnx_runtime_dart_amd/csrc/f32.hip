@@ -377,7 +377,7 @@ int mg_f32_ksplit(int64_t M, int64_t K, int64_t batch) {
 // (ny * pc row tiles of A + nx * pr column tiles of B, equal sizes), then the
 // largest rectangle.  Returns false (row-major order) for grids of fewer than
 // 64 tiles or that no cut fits.
-static bool mg_f32_xcd_cut(int64_t ny, int64_t nx, int *pr, int *pc, int64_t *per) {
+bool mg_f32_xcd_cut(int64_t ny, int64_t nx, int *pr, int *pc, int64_t *per) {
   if (ny * nx < 64) return false;
   int64_t best = -1, best_per = 0;
   for (int r = 1; r <= 8; r *= 2) {

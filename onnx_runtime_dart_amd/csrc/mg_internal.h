@@ -56,6 +56,10 @@ struct mg_ctx {
   // host-pointer calls.  Reused across calls of this context only.
   void *ws = nullptr;
   size_t ws_bytes = 0;
+  // A captured graph may hold the address of ws (mg_ws_optional): a larger
+  // workspace then does not free it; it waits in ws_old for the context's end.
+  bool ws_captured = false;
+  std::vector<void *> ws_old;
   // Compute units of the device (grid sizing).
   int num_cus = 256;
   void *pin = nullptr;  // MG_PIN_SLOTS * MG_PIN_SLOT_BYTES pinned host bytes
@@ -131,6 +135,7 @@ struct mg_int8_dev {
 
 struct mg_f32_dev {
   float *b = nullptr;  // [N][K] row-major (B^T; transposed at upload unless transB)
+  void *pair = nullptr;  // its pair images (mg_pair_split), or null
 };
 
 struct mg_weight {
@@ -149,6 +154,11 @@ struct mg_weight {
 mg_status mg_check_control(mg_ctx *ctx, int64_t additional_bytes);
 // Ensures ctx->ws holds at least `bytes` (grow-only).
 mg_status mg_ws_reserve(mg_ctx *ctx, size_t bytes);
+// Whether an op that can also run with less (or no) workspace may take
+// `bytes` of it: within the byte budget, and there or allocated now.  Under
+// stream capture only a workspace that is already large enough serves (no
+// allocation there), and it then outlives growth for the graph's sake.
+bool mg_ws_optional(mg_ctx *ctx, size_t bytes);
 // Sets the context's device current on this thread.
 mg_status mg_use_device(mg_ctx *ctx);
 // Copies `bytes` of host memory to device memory on the context's stream.
@@ -323,6 +333,18 @@ mg_status mg_f32_run(mg_ctx *ctx, const mg_f32_problem &p, const float *a_dev,
 // only, so column slices of a weight take the same split (bitwise equal
 // columns).
 int mg_f32_ksplit(int64_t M, int64_t K, int64_t batch);
+// The XCD cut of an ny x nx grid of square tiles (see f32.hip); false:
+// row-major.
+bool mg_f32_xcd_cut(int64_t ny, int64_t nx, int *pr, int *pc, int64_t *per);
+
+// Pair images (fp16 hi and lo digits in MFMA order and row exponents, see
+// pair.hip) of an fp32 matrix of R rows of K contiguous elements, and y =
+// alpha A . B^T + beta C of one batch on the images of A [M, K] and B [N, K].
+constexpr int64_t MG_PAIR_MAX_N = 1 << 22;  // 32-bit offsets within an output tile
+size_t mg_pair_bytes(int64_t R, int64_t K);
+mg_status mg_pair_split(mg_ctx *ctx, const float *x_dev, int64_t R, int64_t K, void *img);
+mg_status mg_pair_run(mg_ctx *ctx, const mg_f32_problem &p, const float *a_dev,
+                      const void *a_img, const float *b_dev, const void *b_img, float *y_dev);
 // MatMul on operands given as doubles (the reference's non-float fallback):
 // double products summed in k order, one rounding to f32.  Uses p.M, K, N,
 // batch and bc (row-major A [M, K] and B [K, N] per batch).

@@ -1,0 +1,384 @@
+// fp32 products on fp16 MFMA: operands as pairs of fp16 digits.
+//
+// Every operand row (a row of A, a column of B) is scaled by a power of two
+// that puts its largest magnitude in [2^14, 2^15) and each element x is
+// carried as hi = fp16(x) and lo = fp16((x - hi) 2^11).  hi and lo hold 23
+// significant bits of x (fp32's 24 less half a bit on average) for every
+// element down to 2^-29 of the row's largest, and the smaller ones to 2^-51
+// of it.  The product is hi hi' + 2^-11 (hi lo' + lo hi'), each sum in an
+// fp32 accumulator of its own; lo lo' (2^-24 of the product at most) is left
+// out.  Three v_mfma_f32_32x32x16_f16 take the place of eight
+// v_mfma_f32_32x32x2_f32 on 1/5 of their matrix-core time, and the leading
+// sum is rounded once per 16 k instead of once per 2.
+//
+// Rows that hold Inf or NaN are marked; their outputs are computed on fp32
+// MFMA from the fp32 operands (f32_tile).
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+
+#include "mg_internal.h"
+
+namespace {
+
+typedef float float16v __attribute__((ext_vector_type(16)));
+typedef float float4v __attribute__((ext_vector_type(4)));
+typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+
+constexpr int kMarked = 1 << 29;  // row exponent of a row with Inf or NaN
+
+// The pair of eight fp32 values scaled by 2^e.
+__device__ inline void split8(const float v[8], int e, half8 *hi, half8 *lo) {
+#pragma unroll
+  for (int i = 0; i < 8; i++) {
+    const float x = ldexpf(v[i], e);
+    const _Float16 h = (_Float16)x;
+    (*hi)[i] = h;
+    (*lo)[i] = (_Float16)((x - (float)h) * 2048.f);
+  }
+}
+
+// Pair images of X [R, K] (row-major, K contiguous): per 32 rows and 16 k a
+// hi and a lo fragment of 1 KiB in MFMA operand order, [r32][k16][hi|lo][32 h
+// + r][8] for row r and k = 16 k16 + 8 h .. +7; zeros past R and K.  ex[row]
+// is the row's exponent (kMarked: Inf or NaN, digits zero).
+// TPR threads per row, 256 / TPR rows per workgroup; UL > 0: a thread keeps
+// its UL octets in registers between the row maximum and the split (K <= 8
+// TPR UL), UL = 0 reads the row twice.  Bound by memory at large R (4096 x 1536:
+// 25 MB in, 25 MB out, 10.4 us, 4.8 TB/s) and by its launch and one round trip at small ones, so
+// rows of few workgroups take a whole workgroup each.
+template <int TPR, int UL>
+__global__ __launch_bounds__(256) void k_pair_split(const float *__restrict__ X, int64_t R,
+                                                    int64_t K, int nk, int vec,
+                                                    uint4 *__restrict__ img,
+                                                    int *__restrict__ ex) {
+  const int t = threadIdx.x, u = t % TPR;
+  const int64_t row = (int64_t)blockIdx.x * (256 / TPR) + t / TPR;
+  const float *x = X + row * K;
+  auto load = [&](int o, float v[8]) __attribute__((always_inline)) {
+    const int64_t k0 = (int64_t)o * 8;
+    if (row < R && vec && k0 + 8 <= K) {
+      const float4v a = *reinterpret_cast<const float4v *>(x + k0);
+      const float4v b = *reinterpret_cast<const float4v *>(x + k0 + 4);
+#pragma unroll
+      for (int i = 0; i < 4; i++) v[i] = a[i], v[4 + i] = b[i];
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; i++) v[i] = row < R && k0 + i < K ? x[k0 + i] : 0.f;
+    }
+  };
+  // Largest magnitude as bits: ordered as integers, Inf and NaN largest.
+  unsigned mx = 0;
+  auto amax = [&](const float v[8]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 8; i++) mx = max(mx, __builtin_bit_cast(unsigned, v[i]) & 0x7fffffffu);
+  };
+  const int no = 2 * nk;
+  float v[UL ? UL : 1][8];
+  if constexpr (UL > 0) {
+#pragma unroll
+    for (int j = 0; j < UL; j++) load(u + TPR * j, v[j]);
+#pragma unroll
+    for (int j = 0; j < UL; j++) amax(v[j]);
+  } else {
+    for (int o = u; o < no; o += TPR) {
+      load(o, v[0]);
+      amax(v[0]);
+    }
+  }
+  for (int o = std::min(TPR, 64) / 2; o > 0; o >>= 1) mx = max(mx, (unsigned)__shfl_xor((int)mx, o));
+  if constexpr (TPR > 64) {
+    __shared__ unsigned wmx[4];
+    if ((t & 63) == 0) wmx[t >> 6] = mx;
+    __syncthreads();
+    mx = max(max(wmx[0], wmx[1]), max(wmx[2], wmx[3]));
+  }
+  const bool marked = mx >= 0x7f800000u;
+  int e = 0;
+  if (mx && !marked) {
+    int xp;
+    frexpf(__builtin_bit_cast(float, mx), &xp);
+    e = 15 - xp;
+  }
+  if (u == 0) ex[row] = marked ? kMarked : e;
+  auto store = [&](int o, const float w[8]) __attribute__((always_inline)) {
+    if (o >= no) return;
+    half8 hi = {}, lo = {};
+    if (!marked) split8(w, e, &hi, &lo);
+    uint4 *d = img + (((row >> 5) * nk + (o >> 1)) * 2) * 64 + 32 * (o & 1) + (row & 31);
+    d[0] = __builtin_bit_cast(uint4, hi);
+    d[64] = __builtin_bit_cast(uint4, lo);
+  };
+  if constexpr (UL > 0) {
+#pragma unroll
+    for (int j = 0; j < UL; j++) store(u + TPR * j, v[j]);
+  } else {
+    for (int o = u; o < no; o += TPR) {
+      load(o, v[0]);
+      store(o, v[0]);
+    }
+  }
+}
+
+// One 32 x 32 output tile of A [M, K] . B [N, K]^T on fp32 MFMA (k pairs in
+// order), operands read from memory with bounds checks.
+__device__ inline float16v f32_tile(const float *__restrict__ A, const float *__restrict__ B,
+                                    int64_t M, int64_t N, int64_t K, int64_t r0, int64_t c0,
+                                    int lane) {
+  const int64_t r = r0 + (lane & 31), c = c0 + (lane & 31);
+  float16v acc = {};
+  for (int64_t kb = 0; kb < K; kb += 16) {
+    float a[8], b[8];
+#pragma unroll
+    for (int s = 0; s < 8; s++) {
+      const int64_t k = kb + 2 * s + (lane >> 5);
+      a[s] = r < M && k < K ? A[r * K + k] : 0.f;
+      b[s] = c < N && k < K ? B[c * K + k] : 0.f;
+    }
+#pragma unroll
+    for (int s = 0; s < 8; s++)
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s], b[s], acc, 0, 0, 0);
+  }
+  return acc;
+}
+
+struct PairArgs {
+  const uint4 *ai, *bi;     // pair images
+  const int *ae, *be;       // row exponents
+  const float *a, *b;       // the fp32 operands (marked rows)
+  int64_t M, N, K;
+  int nk, nx, pr, pc;       // 16-k steps; tile grid and its XCD cut
+  float alpha, beta;
+  const float *c;
+  int64_t c_rs, c_cs, ldy;
+  float *y;
+};
+
+// A 64 x 64 workgroup tile, the four waves a quarter of the 16-k steps each,
+// their sums added in wave order through LDS.  Fragments stream from L2
+// straight into registers, two steps in flight.
+// What bounds it is the rate at which a CU takes fragments in (8 KiB per wave
+// and 12 MFMAs; a workgroup alone on a CU gets ~90 GB/s), with launch, first
+// loads and epilogue around it at small sizes.  Measured (4096 x 384 -> 1536
+// / 4096 x 1536 -> 384 / 256 x 2048 -> 512, us a call with the split of A;
+// fp32 MFMA kernel 58 / 57 / 30): this form 30.7 / 31.6 / 19.6; 128 x 128
+// tiles without the K shares 32.1 / 45.8 / 44.8; fragments through an LDS
+// ring of 4 steps, 128 x 128 tiles 31.3 / 45.1 / 46.7 and 64 x 64 tiles 48.3 /
+// 38.9 / 23.2; three steps in flight 31.8 / 32.1 / 19.8.  One form for all
+// sizes also keeps an output's sums independent of M and N: rows and column
+// slices agree bitwise.
+__global__ __launch_bounds__(256, 2) void k_pair_gemm(const PairArgs p) {
+  constexpr int T = 64, KW = 4, D = 2;
+  __shared__ float4v part[KW][4][4][64];  // [wave][32 x 32 block][v / 4][lane]
+  __shared__ __attribute__((aligned(16))) int exps[2 * T];
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  int tr, tc;
+  {
+    const int L = (int)blockIdx.x;
+    if (p.pr == 0) {
+      tr = L / p.nx;
+      tc = L % p.nx;
+    } else {
+      const int ny = (int)((p.M + T - 1) / T);
+      const int x = L & 7, i = L >> 3, br = x / p.pc, bcol = x % p.pc;
+      const int rlo = br * ny / p.pr, rhi = (br + 1) * ny / p.pr;
+      const int clo = bcol * p.nx / p.pc, chi = (bcol + 1) * p.nx / p.pc;
+      const int w = chi - clo;
+      if (i >= (rhi - rlo) * w) return;  // uniform: the whole workgroup leaves
+      tr = rlo + i / w;
+      tc = clo + i % w;
+    }
+  }
+  const int nk = p.nk, per = nk / KW;  // steps; of each wave (nk is a multiple of 4)
+  const int64_t r0 = (int64_t)tr * T, c0 = (int64_t)tc * T;
+  auto rsrc = [](const void *base) __attribute__((always_inline)) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), (short)0, 0x7ffffff0,
+                                             0x00020000);
+  };
+  const __amdgpu_buffer_rsrc_t ra = rsrc(p.ai + (r0 >> 5) * nk * 128);
+  const __amdgpu_buffer_rsrc_t rb = rsrc(p.bi + (c0 >> 5) * nk * 128);
+  half8 a[D][2][2], b[D][2][2];  // [slot][32-row block][hi, lo]
+  auto load = [&](int d, int k) __attribute__((always_inline)) {
+    k = wave * per + min(k, per - 1);
+#pragma unroll
+    for (int g = 0; g < 2; g++)
+#pragma unroll
+      for (int i = 0; i < 2; i++) {
+        a[d][i][g] = __builtin_bit_cast(
+            half8, __builtin_amdgcn_raw_buffer_load_b128(ra, lane * 16 + g * 1024,
+                                                         (i * nk + k) * 2048, 0));
+        b[d][i][g] = __builtin_bit_cast(
+            half8, __builtin_amdgcn_raw_buffer_load_b128(rb, lane * 16 + g * 1024,
+                                                         (i * nk + k) * 2048, 0));
+      }
+  };
+  float16v s1[2][2], s2[2][2];
+#pragma unroll
+  for (int i = 0; i < 4; i++) s1[i >> 1][i & 1] = s2[i >> 1][i & 1] = (float16v){};
+  auto step = [&](int d) __attribute__((always_inline)) {
+#pragma unroll
+    for (int g = 0; g < 3; g++)
+#pragma unroll
+      for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+          float16v &s = g == 0 ? s1[i][j] : s2[i][j];
+          s = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[d][i][g == 2], b[d][j][g == 1], s, 0, 0, 0);
+        }
+  };
+  // The tile's exponents (images reach to whole 64-row blocks) and a column's
+  // C where C is a row: read here, not in the epilogue, where each would be a
+  // round trip of its own.
+  const int l32 = lane & 31, h = lane >> 5;
+  if (t < 2 * T) exps[t] = t < T ? p.ae[r0 + t] : p.be[c0 + t - T];
+  float cb[2] = {0.f, 0.f};
+  if (p.c && p.c_rs == 0)
+#pragma unroll
+    for (int j = 0; j < 2; j++) cb[j] = p.c[min(c0 + 32 * j + l32, p.N - 1) * p.c_cs];
+#pragma unroll
+  for (int d = 0; d < D; d++) load(d, d);
+  __syncthreads();  // exps
+  int k = 0;
+  for (; k + D <= per; k += D) {
+#pragma unroll
+    for (int d = 0; d < D; d++) {
+      step(d);
+      load(d, k + D + d);
+    }
+  }
+#pragma unroll
+  for (int d = 0; d < D; d++)
+    if (k + d < per) step(d);
+  // y = sum 2^-(ea + eb) of the 32 x 32 block (i, j) of the tile: lane
+  // l holds column l % 32 and rows 8 (v / 4) + 4 (l / 32) + v % 4.  Stores
+  // past M or N go past the resource and are dropped in hardware.
+  auto finish = [&](const float16v &sum, int i, int j) __attribute__((always_inline)) {
+    const int64_t tr0 = r0 + 32 * i, tc0 = c0 + 32 * j;
+    if (tr0 >= p.M || tc0 >= p.N) return;
+    const int64_t col = tc0 + l32, rw = tr0 + 4 * h;
+    const int eb = exps[T + 32 * j + l32];
+    int ea[16];
+    bool marked = eb == kMarked;
+#pragma unroll
+    for (int v = 0; v < 16; v += 4) {
+      const int4 x = *reinterpret_cast<const int4 *>(&exps[32 * i + 4 * h + 2 * v]);
+      ea[v] = x.x, ea[v + 1] = x.y, ea[v + 2] = x.z, ea[v + 3] = x.w;
+      marked |= x.x == kMarked || x.y == kMarked || x.z == kMarked || x.w == kMarked;
+    }
+    float16v e = {};
+    if (__builtin_expect(__ballot(marked) != 0, 0))
+      e = f32_tile(p.a, p.b, p.M, p.N, p.K, tr0, tc0, lane);
+    float cv[16];
+#pragma unroll
+    for (int v = 0; v < 16; v++) cv[v] = cb[j];
+    if (p.c && p.c_rs) {
+#pragma unroll
+      for (int v = 0; v < 16; v++) {
+        const int64_t row = rw + 8 * (v >> 2) + (v & 3);
+        cv[v] = p.c[row < p.M && col < p.N ? row * p.c_rs + col * p.c_cs : 0];
+      }
+    }
+    const __amdgpu_buffer_rsrc_t ry = rsrc(p.y + tr0 * p.ldy + tc0);
+#pragma unroll
+    for (int v = 0; v < 16; v++) {
+      const int lr = 4 * h + 8 * (v >> 2) + (v & 3);
+      float y = ldexpf(sum[v], -(ea[v] + eb));
+      if (ea[v] == kMarked || eb == kMarked) y = e[v];
+      if (p.alpha != 1.f) y = p.alpha * y;
+      if (p.c) y = y + (p.beta != 1.f ? p.beta * cv[v] : cv[v]);
+      __builtin_amdgcn_raw_buffer_store_b32(
+          __builtin_bit_cast(unsigned, y), ry,
+          tr0 + lr < p.M && col < p.N ? (unsigned)(lr * (int)p.ldy + l32) * 4u : 0x80000000u, 0, 0);
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+#pragma unroll
+      for (int v = 0; v < 16; v++) s1[i][j][v] = fmaf(s2[i][j][v], 1.f / 2048.f, s1[i][j][v]);
+#pragma unroll
+  for (int q = 0; q < 4; q++)
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      const float16v &s = s1[q >> 1][q & 1];
+      part[wave][q][v][lane] = (float4v){s[4 * v], s[4 * v + 1], s[4 * v + 2], s[4 * v + 3]};
+    }
+  __syncthreads();
+  // Wave q finishes block q.
+  float16v sum;
+#pragma unroll
+  for (int v = 0; v < 4; v++) {
+    float4v x = part[0][wave][v][lane];
+#pragma unroll
+    for (int w = 1; w < KW; w++) x += part[w][wave][v][lane];
+#pragma unroll
+    for (int e = 0; e < 4; e++) sum[4 * v + e] = x[e];
+  }
+  finish(sum, wave >> 1, wave & 1);
+}
+
+}  // namespace
+
+// 16-k steps of the images: K padded with zeros to a multiple of 64 k, so
+// that the K shares of a tile's waves are equal.
+static int64_t mg_pair_steps(int64_t K) { return (K + 63) / 64 * 4; }
+
+size_t mg_pair_bytes(int64_t R, int64_t K) {
+  const int64_t r = (R + 63) / 64 * 64, nk = mg_pair_steps(K);
+  return mg_align((size_t)(r * nk * 64)) + mg_align((size_t)r * 4);
+}
+
+mg_status mg_pair_split(mg_ctx *ctx, const float *x_dev, int64_t R, int64_t K, void *img) {
+  const int64_t rp = (R + 63) / 64 * 64;
+  const int nk = (int)mg_pair_steps(K);
+  uint4 *im = static_cast<uint4 *>(img);
+  int *ex = reinterpret_cast<int *>(static_cast<char *>(img) + mg_align((size_t)(rp * nk * 64)));
+  const int vec = reinterpret_cast<uintptr_t>(x_dev) % 16 == 0 && K % 4 == 0;
+#define MG_SPLIT(TPR, UL)                                                                    \
+  hipLaunchKernelGGL((k_pair_split<TPR, UL>), dim3((unsigned)(rp / (256 / TPR))), dim3(256), 0, \
+                     ctx->stream, x_dev, R, K, nk, vec, im, ex)
+  if (rp * K >= (int64_t)1 << 20 && K <= 2048) {
+    if (K <= 512) MG_SPLIT(32, 2);
+    else if (K <= 1024) MG_SPLIT(32, 4);
+    else MG_SPLIT(32, 8);
+  } else {
+    if (K <= 2048) MG_SPLIT(256, 1);
+    else if (K <= 8192) MG_SPLIT(256, 4);
+    else MG_SPLIT(256, 0);
+  }
+#undef MG_SPLIT
+  return mg_launch_check("k_pair_split");
+}
+
+mg_status mg_pair_run(mg_ctx *ctx, const mg_f32_problem &p, const float *a_dev,
+                      const void *a_img, const float *b_dev, const void *b_img, float *y_dev) {
+  const int64_t mp = (p.M + 63) / 64 * 64, np = (p.N + 63) / 64 * 64;
+  PairArgs q{};
+  q.nk = (int)mg_pair_steps(p.K);
+  q.ai = static_cast<const uint4 *>(a_img);
+  q.bi = static_cast<const uint4 *>(b_img);
+  q.ae = reinterpret_cast<const int *>(static_cast<const char *>(a_img) + mg_align((size_t)(mp * q.nk * 64)));
+  q.be = reinterpret_cast<const int *>(static_cast<const char *>(b_img) + mg_align((size_t)(np * q.nk * 64)));
+  q.a = a_dev;
+  q.b = b_dev;
+  q.M = p.M;
+  q.N = p.N;
+  q.K = p.K;
+  q.alpha = p.alpha;
+  q.beta = p.beta;
+  q.c = p.c;
+  q.c_rs = p.c_rs;
+  q.c_cs = p.c_cs;
+  q.ldy = p.ldy ? p.ldy : p.N;
+  q.y = y_dev;
+  const int64_t nx = np / 64, ny = mp / 64;
+  q.nx = (int)nx;
+  int64_t per = 0;
+  const bool cut = mg_f32_xcd_cut(ny, nx, &q.pr, &q.pc, &per);
+  if (!cut) q.pr = q.pc = 0;
+  const unsigned gx = (unsigned)(cut ? 8 * per : nx * ny);
+  hipLaunchKernelGGL(k_pair_gemm, dim3(gx), dim3(256), 0, ctx->stream, q);
+  return mg_launch_check("k_pair_gemm");
+}

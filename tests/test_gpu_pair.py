@@ -1,0 +1,107 @@
+"""Weight Gemms on fp16 digit pairs (F32Weight.gemm) against float64, at the
+edges of their 64 x 64 tiles and 64-k padding, over every plan of the digit
+split, over wide exponent ranges, with Inf and NaN operands (the fp32 form of
+the tile) and without the workspace they would like to have (the fp32 MFMA
+kernel)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from onnx_runtime_dart_amd import ops as _ops
+    return _ops
+
+
+def check(y, a, w, c=0.0, alpha=1.0, beta=1.0):
+    """Element by element: the two digits leave 2^-23 of an operand, lo lo'
+    2^-24 of a product, and each of the K / 16 additions per output (and the
+    few that join the shares, scale and add C) at most 2^-23 of what has been
+    added, all of it at most sum |a| |w|."""
+    a, w = a.astype(np.float64), w.astype(np.float64)
+    want = alpha * (a @ w.T) + beta * c
+    size = abs(alpha) * (np.abs(a) @ np.abs(w).T) + np.abs(beta * c)
+    bound = (a.shape[1] / 16 + 12) * 2.0**-23 * size + 2.0**-148
+    assert (np.abs(y - want) <= bound).all()
+
+
+@pytest.mark.parametrize("m,k,n", [(1, 1, 1), (63, 15, 65), (65, 64, 63), (64, 65, 64),
+                                   (1, 2049, 130), (130, 8200, 70), (2049, 513, 65),
+                                   (1030, 1025, 33), (700, 1537, 129), (4096, 384, 200)])
+def test_tile_edges(ops, m, k, n):
+    rng = np.random.default_rng(m + k + n)
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    w = rng.standard_normal((n, k)).astype(np.float32)
+    fw = ops.F32Weight(w, trans_b=True)
+    check(fw.gemm(a), a, w)
+    bias = rng.standard_normal(n).astype(np.float32)
+    check(fw.gemm(a, bias, alpha=0.5, beta=2.0), a, w, bias, 0.5, 2.0)
+    full = rng.standard_normal((m, n)).astype(np.float32)
+    check(fw.gemm(a, full), a, w, full)
+    col = rng.standard_normal((m, 1)).astype(np.float32)
+    check(fw.gemm(a, col), a, w, col)
+    fw.release()
+
+
+def test_exponent_ranges(ops):
+    # Rows and columns from 2^-140 to 2^60, elements of a row over 2^40, zeros.
+    rng = np.random.default_rng(3)
+    a = rng.standard_normal((70, 200)) * 2.0 ** rng.integers(-20, 21, (70, 200))
+    a *= 2.0 ** np.linspace(-120, 60, 70)[:, None]
+    a[5] = 0
+    w = rng.standard_normal((66, 200)) * 2.0 ** np.linspace(-60, 40, 66)[:, None]
+    w[7] = 0
+    a, w = a.astype(np.float32), w.astype(np.float32)
+    fw = ops.F32Weight(w, trans_b=True)
+    check(fw.gemm(a), a, w)
+    fw.release()
+
+
+def test_inf_and_nan(ops):
+    # An Inf or NaN touches its own row's (column's) outputs, as the sum in
+    # fp32 gives them; the other outputs are those without it.
+    rng = np.random.default_rng(4)
+    a = rng.standard_normal((100, 150)).astype(np.float32)
+    w = rng.standard_normal((90, 150)).astype(np.float32)
+    fw = ops.F32Weight(w, trans_b=True)
+    clean = fw.gemm(a)
+    b = a.copy()
+    b[3, 7], b[40, 100], b[77, 149], b[77, 0] = np.inf, np.nan, -np.inf, np.inf
+    y = fw.gemm(b)
+    fw.release()
+    rows = np.setdiff1d(np.arange(100), [3, 40, 77])
+    np.testing.assert_array_equal(y[rows], clean[rows])
+    np.testing.assert_array_equal(y[3], np.sign(w[:, 7]) * np.float32(np.inf))
+    assert np.isnan(y[40]).all()
+    same = np.sign(w[:, 149]) == -np.sign(w[:, 0])
+    np.testing.assert_array_equal(np.isnan(y[77]), ~same)
+    v = w.copy()
+    v[11, 2], v[64, 64] = np.inf, np.nan
+    fw = ops.F32Weight(v, trans_b=True)
+    z = fw.gemm(a)
+    fw.release()
+    cols = np.setdiff1d(np.arange(90), [11, 64])
+    np.testing.assert_array_equal(z[:, cols], clean[:, cols])
+    np.testing.assert_array_equal(z[:, 11], np.sign(a[:, 2]) * np.float32(np.inf))
+    assert np.isnan(z[:, 64]).all()
+
+
+def test_without_workspace(ops):
+    # A byte budget below the images of A: the call still runs (fp32 MFMA).
+    rng = np.random.default_rng(5)
+    a = rng.standard_normal((70, 96)).astype(np.float32)
+    w = rng.standard_normal((40, 96)).astype(np.float32)
+    ctx = ops.default_context()
+    fw = ops.F32Weight(w, trans_b=True, ctx=ctx)
+    ad, yd = ops.DeviceBuffer.from_array(a), ops.DeviceBuffer(70 * 40 * 4)
+    ctx.set_control(None, max_bytes=64)
+    try:
+        fw.gemm_dev(ad.ptr, 70, yd.ptr)
+    finally:
+        ctx.set_control(None, max_bytes=-1)
+    check(yd.to_array((70, 40), np.float32), a, w)
+    for b in (ad, yd):
+        b.free()
+    fw.release()
