@@ -1,0 +1,371 @@
+// fp32 Conv (one group) as an implicit GEMM on fp16 digit pairs
+// (pair_common.h): lib/src/onnx_nn_ops.dart:179-817.
+//
+// Rows of the product are the output channels (the filters, scaled by a power
+// of two per channel), columns the output positions of all images (the input,
+// scaled per image), k = (16-channel block, tap).  Two launches lay the
+// operands out:
+//   * k_conv_pair_prep: the filters' pair fragments, [m32][step][hi|lo][lane]
+//     with step = block * taps + tap, and the largest magnitude of each chunk
+//     of each image;
+//   * k_conv_pair_x: the input as [image][block][hi|lo][position][16] with the
+//     padding written out as zeros, a position being one of the padded window.
+// So a step's operand of 32 consecutive output positions is 32-byte pieces
+// at the positions' window origins (one 32-bit offset per lane, the same in
+// every step) plus the step's own offset, a scalar: the products' loop has
+// no gather arithmetic, no masks and no LDS.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+
+#include "pair_common.h"
+
+namespace {
+
+constexpr int kMaxChunks = 64;  // chunk maxima per image (one per lane of a wave)
+
+struct ConvPair {
+  const float *x, *w, *bias;
+  float *y;
+  int n, c, m, taps, cb, ns;      // images, channels, 16-channel blocks, steps (padded to 4)
+  int in[3], out[3], ker[3], str[3], dil[3], pad[3], win[3];  // win: padded window dims
+  int in_sp, out_sp, win_sp;
+  int chunks, chunk;              // maxima chunks of an image, elements of each
+  uint4 *wi, *xi;                 // images of the filters and of the input
+  int *we, *xe;                   // their exponents
+  unsigned *part;                 // [n][chunks] largest magnitudes (bits)
+  int nx, pr, pc;                 // tile grid and its XCD cut
+};
+
+// Bound by latency (a few loads per thread, one round trip each way): the
+// filters' rows and the input's maxima share one launch.
+__global__ __launch_bounds__(256) void k_conv_pair_prep(const ConvPair p) {
+  const int t = threadIdx.x;
+  const int mp = (p.m + 63) / 64 * 64;
+  const bool filt = (int)blockIdx.x < mp;
+  const int m = blockIdx.x, K = p.c * p.taps;
+  const int q = (int)blockIdx.x - mp, img = filt ? 0 : q / p.chunks, ch = q - img * p.chunks;
+  const int64_t xn = (int64_t)p.c * p.in_sp;
+  const float *src = filt ? p.w + (int64_t)m * K : p.x + img * xn + (int64_t)ch * p.chunk;
+  const int len = filt ? (m < p.m ? K : 0)
+                       : (int)std::min<int64_t>(p.chunk, xn - (int64_t)ch * p.chunk);
+  unsigned mx = 0;
+  for (int i = t; i < len; i += 8 * 256) {
+    float v[8];
+#pragma unroll
+    for (int u = 0; u < 8; u++) v[u] = src[min(i + 256 * u, len - 1)];
+#pragma unroll
+    for (int u = 0; u < 8; u++) mx = max(mx, __builtin_bit_cast(unsigned, v[u]) & 0x7fffffffu);
+  }
+  for (int o = 32; o > 0; o >>= 1) mx = max(mx, (unsigned)__shfl_xor((int)mx, o));
+  __shared__ unsigned wmx[4];
+  if ((t & 63) == 0) wmx[t >> 6] = mx;
+  __syncthreads();
+  mx = max(max(wmx[0], wmx[1]), max(wmx[2], wmx[3]));
+  if (!filt) {
+    if (t == 0) p.part[q] = mx;
+    return;
+  }
+  const int e = pair_exponent(mx);
+  if (t == 0) p.we[m] = e;
+  // Octet o: channels 8 c8 .. +7 of tap r, then the padding steps' zeros.
+  const int real = p.cb * p.taps;
+  for (int o = t; o < 2 * p.ns; o += 256) {
+    const int c8 = o / p.taps, r = o - c8 * p.taps;
+    float v[8] = {};
+    if (o < 2 * real && m < p.m)
+#pragma unroll
+      for (int j = 0; j < 8; j++)
+        if (8 * c8 + j < p.c) v[j] = src[(8 * c8 + j) * p.taps + r];
+    half8 hi, lo;
+    pair_split8(v, e, &hi, &lo);
+    const int s = o < 2 * real ? (c8 >> 1) * p.taps + r : o >> 1, h = o < 2 * real ? c8 & 1 : o & 1;
+    uint4 *d = p.wi + ((int64_t)(m >> 5) * p.ns + s) * 128 + 32 * h + (m & 31);
+    d[0] = __builtin_bit_cast(uint4, hi);
+    d[64] = __builtin_bit_cast(uint4, lo);
+  }
+}
+
+// Thread = one position of the padded window, 16 channels (grid: positions,
+// channel blocks, images).  Bound by memory at large inputs.
+__global__ __launch_bounds__(256) void k_conv_pair_x(const ConvPair p) {
+  const int t = threadIdx.x, lane = t & 63;
+  const int pos = (int)blockIdx.x * 256 + t, cb = blockIdx.y, img = blockIdx.z;
+  const int zx = pos % p.win[2], zy = pos / p.win[2] % p.win[1], zz = pos / p.win[2] / p.win[1];
+  const int ix = zx - p.pad[2], iy = zy - p.pad[1], iz = zz - p.pad[0];
+  const bool in = pos < p.win_sp && (unsigned)ix < (unsigned)p.in[2] &&
+                  (unsigned)iy < (unsigned)p.in[1] && (unsigned)iz < (unsigned)p.in[0];
+  const int c0 = 16 * cb;
+  const float *src = p.x + ((int64_t)img * p.c + c0) * p.in_sp +
+                     (in ? (iz * p.in[1] + iy) * p.in[2] + ix : 0);
+  float v[2][8];
+#pragma unroll
+  for (int j = 0; j < 16; j++) v[j >> 3][j & 7] = src[(int64_t)min(j, p.c - 1 - c0) * p.in_sp];
+  unsigned mx = lane < p.chunks ? p.part[img * p.chunks + lane] : 0;
+  for (int o = 32; o > 0; o >>= 1) mx = max(mx, (unsigned)__shfl_xor((int)mx, o));
+  const int e = pair_exponent(mx);
+  if (pos == 0 && cb == 0) p.xe[img] = e;
+  if (pos >= p.win_sp) return;
+  uint4 *d = p.xi + ((int64_t)img * p.cb + cb) * p.win_sp * 4 + 2 * pos;
+#pragma unroll
+  for (int h = 0; h < 2; h++) {
+#pragma unroll
+    for (int j = 0; j < 8; j++)
+      if (!in || c0 + 8 * h + j >= p.c) v[h][j] = 0.f;
+    half8 hi, lo;
+    pair_split8(v[h], e, &hi, &lo);
+    d[h] = __builtin_bit_cast(uint4, hi);
+    d[2 * p.win_sp + h] = __builtin_bit_cast(uint4, lo);
+  }
+}
+
+// The 32 x 32 block of channels m0 .. and columns of which lane l's is (img,
+// window origin oz, oy, ox), on fp32 MFMA straight from the tensors (marked
+// filters or images).
+__device__ inline float16v conv_f32_tile(const ConvPair &p, int m0, int img, int oz, int oy, int ox,
+                                         int lane) {
+  const int m = m0 + (lane & 31), K = p.c * p.taps;
+  float16v acc = {};
+  for (int k0 = 0; k0 < K; k0 += 2) {
+    const int k = k0 + (lane >> 5);
+    const int c = k / p.taps, r = k - c * p.taps;
+    const int kx = r % p.ker[2], ky = r / p.ker[2] % p.ker[1], kz = r / p.ker[2] / p.ker[1];
+    const int iz = oz + kz * p.dil[0], iy = oy + ky * p.dil[1], ix = ox + kx * p.dil[2];
+    const bool ok = k < K && (unsigned)iz < (unsigned)p.in[0] && (unsigned)iy < (unsigned)p.in[1] &&
+                    (unsigned)ix < (unsigned)p.in[2];
+    const float a = k < K && m < p.m ? p.w[(int64_t)m * K + k] : 0.f;
+    const float b =
+        ok ? p.x[((int64_t)img * p.c + c) * p.in_sp + (iz * p.in[1] + iy) * p.in[2] + ix] : 0.f;
+    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, acc, 0, 0, 0);
+  }
+  return acc;
+}
+
+// 64 channels x 64 output positions per workgroup, the four waves a quarter
+// of the steps each (pair_sums).  Bound by the rate at which a CU takes in
+// fragments.  ResNet-50 3 x 3 (32 x 256 x 14 x 14 -> 256): 30 us and 47 with
+// the two launches ahead of it (153 on k_conv's fp32 MFMA, whose gather and
+// fp32 matrix rate bounded it); 16 x 240 x 28 x 28 -> 240: 256 -> 70 us.
+__global__ __launch_bounds__(256, 2) void k_conv_pair(const ConvPair p) {
+  __shared__ float4v part[4][4][4][64];
+  __shared__ int exps[64];
+  __shared__ float bias[64];
+  const int t = threadIdx.x, lane = t & 63, l32 = lane & 31, h = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  int tr, tc;
+  {
+    const int L = (int)blockIdx.x;
+    if (p.pr == 0) {
+      tr = L / p.nx;
+      tc = L % p.nx;
+    } else {
+      const int ny = (p.m + 63) / 64;
+      const int x = L & 7, i = L >> 3, br = x / p.pc, bcol = x % p.pc;
+      const int rlo = br * ny / p.pr, rhi = (br + 1) * ny / p.pr;
+      const int clo = bcol * p.nx / p.pc, chi = (bcol + 1) * p.nx / p.pc;
+      const int w = chi - clo;
+      if (i >= (rhi - rlo) * w) return;  // uniform: the whole workgroup leaves
+      tr = rlo + i / w;
+      tc = clo + i % w;
+    }
+  }
+  const int m0 = tr * 64, cols = p.n * p.out_sp, ns = p.ns, per = ns / 4;
+  if (t < 64) {
+    exps[t] = p.we[m0 + t];
+    bias[t] = p.bias && m0 + t < p.m ? p.bias[m0 + t] : 0.f;
+  }
+  // The lane's column in each of the tile's two 32-column blocks: image,
+  // output position and window origin.
+  int col[2], img[2], pos[2], oz[2], oy[2], ox[2], eb[2];
+  unsigned vb[2];
+#pragma unroll
+  for (int j = 0; j < 2; j++) {
+    col[j] = tc * 64 + 32 * j + l32;
+    const int cc = min(col[j], cols - 1);
+    img[j] = cc / p.out_sp;
+    pos[j] = cc - img[j] * p.out_sp;
+    ox[j] = pos[j] % p.out[2] * p.str[2];
+    oy[j] = pos[j] / p.out[2] % p.out[1] * p.str[1];
+    oz[j] = pos[j] / p.out[2] / p.out[1] * p.str[0];
+    eb[j] = p.xe[img[j]];
+    vb[j] = (unsigned)(img[j] * p.cb * p.win_sp * 64 +
+                       ((oz[j] * p.win[1] + oy[j]) * p.win[2] + ox[j]) * 32 + 16 * h);
+  }
+  auto rsrc = [](const void *base) __attribute__((always_inline)) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), (short)0, 0x7ffffff0,
+                                             0x00020000);
+  };
+  const __amdgpu_buffer_rsrc_t rw = rsrc(p.wi + (int64_t)(m0 >> 5) * ns * 128), rx = rsrc(p.xi);
+  // This wave's next step: 16-channel block and tap; a padding step reads the
+  // last real one (its filters are zero).
+  const int s0 = min(wave * per, p.cb * p.taps - 1);
+  int kb = s0 / p.taps, r0 = s0 % p.taps;
+  int kx = r0 % p.ker[2], ky = r0 / p.ker[2] % p.ker[1], kz = r0 / p.ker[2] / p.ker[1];
+  int at = -1;
+  half8 a[2][2][2], b[2][2][2];
+  auto load = [&](int d, int k) __attribute__((always_inline)) {
+    if (k != at && at >= 0) {
+      if (++kx == p.ker[2]) {
+        kx = 0;
+        if (++ky == p.ker[1]) {
+          ky = 0;
+          if (++kz == p.ker[0]) kz = 0, kb = min(kb + 1, p.cb - 1);
+        }
+      }
+    }
+    at = k;
+    const int so = (kb * 2 * p.win_sp +
+                    (kz * p.dil[0] * p.win[1] + ky * p.dil[1]) * p.win[2] + kx * p.dil[2]) * 32;
+#pragma unroll
+    for (int g = 0; g < 2; g++)
+#pragma unroll
+      for (int i = 0; i < 2; i++) {
+        a[d][i][g] = __builtin_bit_cast(
+            half8, __builtin_amdgcn_raw_buffer_load_b128(
+                       rw, lane * 16 + g * 1024, (i * ns + wave * per + k) * 2048, 0));
+        b[d][i][g] = __builtin_bit_cast(
+            half8, __builtin_amdgcn_raw_buffer_load_b128(rx, vb[i], so + g * p.win_sp * 32, 0));
+      }
+  };
+  float16v s1[2][2];
+  pair_sums(a, b, per, s1, load);
+  // (The barrier of the sum also publishes exps and bias.)
+  const float16v sum = pair_reduce(part, wave, lane, s1);
+  const int i = wave >> 1, j = wave & 1;
+  if (m0 + 32 * i >= p.m || tc * 64 + 32 * j >= cols) return;
+  const int cj = j ? col[1] : col[0], ij = j ? img[1] : img[0], pj = j ? pos[1] : pos[0];
+  const int ej = j ? eb[1] : eb[0];
+  bool marked = ej == kMarked;
+  int ea[16];
+#pragma unroll
+  for (int v = 0; v < 16; v++) {
+    ea[v] = exps[32 * i + 4 * h + 8 * (v >> 2) + (v & 3)];
+    marked |= ea[v] == kMarked;
+  }
+  float16v e = {};
+  if (__builtin_expect(__ballot(marked) != 0, 0))
+    e = conv_f32_tile(p, m0 + 32 * i, ij, (j ? oz[1] : oz[0]) - p.pad[0],
+                      (j ? oy[1] : oy[0]) - p.pad[1], (j ? ox[1] : ox[0]) - p.pad[2], lane);
+  const __amdgpu_buffer_rsrc_t ry = rsrc(p.y);
+#pragma unroll
+  for (int v = 0; v < 16; v++) {
+    const int lr = 32 * i + 4 * h + 8 * (v >> 2) + (v & 3);
+    float y = ldexpf(sum[v], -(ea[v] + ej));
+    if (ea[v] == kMarked || ej == kMarked) y = e[v];
+    if (p.bias) y += bias[lr];
+    __builtin_amdgcn_raw_buffer_store_b32(
+        __builtin_bit_cast(unsigned, y), ry,
+        m0 + lr < p.m && cj < cols ? (unsigned)((ij * p.m + m0 + lr) * p.out_sp + pj) * 4u
+                                   : 0x80000000u,
+        0, 0);
+  }
+}
+
+struct Plan {
+  bool ok = false;
+  ConvPair q{};
+  int64_t nb = 0;  // images per round of launches
+  size_t off_we = 0, off_xi = 0, off_xe = 0, off_part = 0, total = 0;
+};
+
+Plan plan(const mg_conv_problem &p) {
+  Plan r;
+  if (p.xk != MG_CONV_F32 || p.trans || p.phased || p.group != 1) return r;
+  const int64_t lim = (int64_t)1 << 29;
+  int64_t win = 1, out = 1, in = 1, taps = 1;
+  ConvPair &q = r.q;
+  for (int d = 0; d < 3; d++) {
+    const int64_t e = (p.out[d] - 1) * p.str[d] + (p.ker[d] - 1) * p.dil[d] + 1;
+    if (p.dil[d] < 1 || p.str[d] < 1 || p.ker[d] < 1 || p.in[d] < 1 || p.out[d] < 1 || e >= lim ||
+        p.in[d] >= lim || p.pad[d] >= lim || p.pad[d] <= -lim || p.dil[d] >= lim || p.str[d] >= lim)
+      return r;
+    win *= e, out *= p.out[d], in *= p.in[d], taps *= p.ker[d];
+    if (win >= lim || out >= lim || in >= lim || taps >= lim) return r;
+    q.in[d] = (int)p.in[d], q.out[d] = (int)p.out[d], q.ker[d] = (int)p.ker[d];
+    q.str[d] = (int)p.str[d], q.dil[d] = (int)p.dil[d], q.pad[d] = (int)p.pad[d];
+    q.win[d] = (int)e;
+  }
+  if (p.c < 1 || p.c >= lim || p.m < 1 || p.m >= lim || p.n < 1) return r;
+  const int64_t cb = (p.c + 15) / 16, ns = (cb * taps + 3) / 4 * 4, mp = (p.m + 63) / 64 * 64;
+  const int64_t img = cb * win * 64;  // bytes of one image's pairs
+  // Where it pays (us a call here / on k_conv; input [n, c, size, size], m
+  // channels, kernel).  Short sums stay on k_conv, whose one launch costs a
+  // stage per 32 k: [4, 24, 28] 3 x 3 to 64 channels 16.1 / 15.3, [4, 64, 14]
+  // 1 x 1 18 / 13, [2, 256, 14] 1 x 1 16.0 / 16.3, [1, 512, 7] 1 x 1 16.0 /
+  // 28.1.  So do inputs of several times the caches' reach that meet few
+  // products (they pass through memory three times here): [32, 256, 56] 1 x 1
+  // to 64 channels 99 / 67, to 256 of [32, 1024, 14] 35 / 74; and channel
+  // counts that the blocks of 16 more than double ([32, 3, 224] 7 x 7: 206 /
+  // 153).
+  if (p.c * taps < 256 || 16 * cb > 2 * p.c ||
+      (p.m * taps < 128 && p.n * p.c * in * 4 > (int64_t)8 << 20))
+    return r;
+  // 32-bit offsets throughout, and the filter rows as laid out.
+  if (p.w_ms != p.c * taps || p.w_cs != taps || p.c * taps >= lim || p.c * in >= lim ||
+      mp * ns * 64 >= 4 * lim || ns * 2048 * 2 >= 4 * lim || img >= 4 * lim || p.m * out >= lim ||
+      (win + 255) / 256 > 0x7fffff || cb > 65535)
+    return r;
+  const int64_t fit = std::min<int64_t>((64ll << 20) / img, lim / (p.m * out));
+  r.nb = std::max<int64_t>(1, std::min<int64_t>(p.n, std::min<int64_t>(fit, 65535)));
+  q.c = (int)p.c, q.m = (int)p.m, q.taps = (int)taps, q.cb = (int)cb, q.ns = (int)ns;
+  q.in_sp = (int)in, q.out_sp = (int)out, q.win_sp = (int)win;
+  // Chunks of at least 4096 elements, at most kMaxChunks of them.
+  q.chunks = (int)std::min<int64_t>(kMaxChunks, (p.c * in + 4095) / 4096);
+  q.chunk = (int)((p.c * in + q.chunks - 1) / q.chunks);
+  q.chunks = (int)((p.c * in + q.chunk - 1) / q.chunk);
+  if (mp + r.nb * q.chunks >= 0x7fffffff) return r;
+  size_t off = mg_align((size_t)(mp * ns * 64));
+  r.off_we = off;
+  off += mg_align((size_t)mp * 4);
+  r.off_xi = off;
+  off += mg_align((size_t)(r.nb * img));
+  r.off_xe = off;
+  off += mg_align((size_t)r.nb * 4);
+  r.off_part = off;
+  off += mg_align((size_t)(r.nb * q.chunks) * 4);
+  r.total = off;
+  r.ok = true;
+  return r;
+}
+
+}  // namespace
+
+size_t mg_conv_pair_bytes(const mg_conv_problem &p) {
+  const Plan r = plan(p);
+  return r.ok ? r.total : 0;
+}
+
+mg_status mg_conv_pair_run(mg_ctx *ctx, const mg_conv_problem &p, void *ws) {
+  Plan r = plan(p);
+  ConvPair &q = r.q;
+  char *base = static_cast<char *>(ws);
+  q.w = static_cast<const float *>(p.w);
+  q.bias = static_cast<const float *>(p.bias);
+  q.wi = reinterpret_cast<uint4 *>(base);
+  q.we = reinterpret_cast<int *>(base + r.off_we);
+  q.xi = reinterpret_cast<uint4 *>(base + r.off_xi);
+  q.xe = reinterpret_cast<int *>(base + r.off_xe);
+  q.part = reinterpret_cast<unsigned *>(base + r.off_part);
+  const int mp = (q.m + 63) / 64 * 64;
+  for (int64_t n0 = 0; n0 < p.n; n0 += r.nb) {
+    q.n = (int)std::min(r.nb, p.n - n0);
+    q.x = static_cast<const float *>(p.x) + n0 * q.c * q.in_sp;
+    q.y = static_cast<float *>(p.y) + n0 * q.m * q.out_sp;
+    hipLaunchKernelGGL(k_conv_pair_prep, dim3((unsigned)(mp + q.n * q.chunks)), dim3(256), 0,
+                       ctx->stream, q);
+    MG_TRY(mg_launch_check("k_conv_pair_prep"));
+    hipLaunchKernelGGL(k_conv_pair_x,
+                       dim3((unsigned)((q.win_sp + 255) / 256), (unsigned)q.cb, (unsigned)q.n),
+                       dim3(256), 0, ctx->stream, q);
+    MG_TRY(mg_launch_check("k_conv_pair_x"));
+    const int64_t nx = ((int64_t)q.n * q.out_sp + 63) / 64, ny = mp / 64;
+    int64_t per = 0;
+    q.nx = (int)nx;
+    const bool cut = mg_f32_xcd_cut(ny, nx, &q.pr, &q.pc, &per);
+    if (!cut) q.pr = q.pc = 0;
+    hipLaunchKernelGGL(k_conv_pair, dim3((unsigned)(cut ? 8 * per : nx * ny)), dim3(256), 0,
+                       ctx->stream, q);
+    MG_TRY(mg_launch_check("k_conv_pair"));
+  }
+  return MG_OK;
+}

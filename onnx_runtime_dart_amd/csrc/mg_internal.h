@@ -422,6 +422,10 @@ size_t mg_conv_ws_bytes(const mg_conv_problem &p);
 // group), which takes the weight zero points from w_zp_host, not w_zp.
 bool mg_conv_int8_route(const mg_conv_problem &p);
 mg_status mg_conv_run(mg_ctx *ctx, const mg_conv_problem &p, void *ws);
+// fp32 Conv on fp16 digit pairs (conv_pair.hip): the workspace it needs (0:
+// the problem does not take this route), and its launches.
+size_t mg_conv_pair_bytes(const mg_conv_problem &p);
+mg_status mg_conv_pair_run(mg_ctx *ctx, const mg_conv_problem &p, void *ws);
 
 // ---------------------------------------------------------- attention entry
 

@@ -17,26 +17,9 @@
 
 #include <algorithm>
 
-#include "mg_internal.h"
+#include "pair_common.h"
 
 namespace {
-
-typedef float float16v __attribute__((ext_vector_type(16)));
-typedef float float4v __attribute__((ext_vector_type(4)));
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-
-constexpr int kMarked = 1 << 29;  // row exponent of a row with Inf or NaN
-
-// The pair of eight fp32 values scaled by 2^e.
-__device__ inline void split8(const float v[8], int e, half8 *hi, half8 *lo) {
-#pragma unroll
-  for (int i = 0; i < 8; i++) {
-    const float x = ldexpf(v[i], e);
-    const _Float16 h = (_Float16)x;
-    (*hi)[i] = h;
-    (*lo)[i] = (_Float16)((x - (float)h) * 2048.f);
-  }
-}
 
 // Pair images of X [R, K] (row-major, K contiguous): per 32 rows and 16 k a
 // hi and a lo fragment of 1 KiB in MFMA operand order, [r32][k16][hi|lo][32 h
@@ -93,18 +76,12 @@ __global__ __launch_bounds__(256) void k_pair_split(const float *__restrict__ X,
     __syncthreads();
     mx = max(max(wmx[0], wmx[1]), max(wmx[2], wmx[3]));
   }
-  const bool marked = mx >= 0x7f800000u;
-  int e = 0;
-  if (mx && !marked) {
-    int xp;
-    frexpf(__builtin_bit_cast(float, mx), &xp);
-    e = 15 - xp;
-  }
-  if (u == 0) ex[row] = marked ? kMarked : e;
+  const int e = pair_exponent(mx);
+  if (u == 0) ex[row] = e;
   auto store = [&](int o, const float w[8]) __attribute__((always_inline)) {
     if (o >= no) return;
-    half8 hi = {}, lo = {};
-    if (!marked) split8(w, e, &hi, &lo);
+    half8 hi, lo;
+    pair_split8(w, e, &hi, &lo);
     uint4 *d = img + (((row >> 5) * nk + (o >> 1)) * 2) * 64 + 32 * (o & 1) + (row & 31);
     d[0] = __builtin_bit_cast(uint4, hi);
     d[64] = __builtin_bit_cast(uint4, lo);
@@ -168,7 +145,7 @@ struct PairArgs {
 // sizes also keeps an output's sums independent of M and N: rows and column
 // slices agree bitwise.
 __global__ __launch_bounds__(256, 2) void k_pair_gemm(const PairArgs p) {
-  constexpr int T = 64, KW = 4, D = 2;
+  constexpr int T = 64, KW = 4;
   __shared__ float4v part[KW][4][4][64];  // [wave][32 x 32 block][v / 4][lane]
   __shared__ __attribute__((aligned(16))) int exps[2 * T];
   const int t = threadIdx.x, lane = t & 63;
@@ -198,9 +175,9 @@ __global__ __launch_bounds__(256, 2) void k_pair_gemm(const PairArgs p) {
   };
   const __amdgpu_buffer_rsrc_t ra = rsrc(p.ai + (r0 >> 5) * nk * 128);
   const __amdgpu_buffer_rsrc_t rb = rsrc(p.bi + (c0 >> 5) * nk * 128);
-  half8 a[D][2][2], b[D][2][2];  // [slot][32-row block][hi, lo]
+  half8 a[2][2][2], b[2][2][2];
   auto load = [&](int d, int k) __attribute__((always_inline)) {
-    k = wave * per + min(k, per - 1);
+    k += wave * per;
 #pragma unroll
     for (int g = 0; g < 2; g++)
 #pragma unroll
@@ -213,20 +190,6 @@ __global__ __launch_bounds__(256, 2) void k_pair_gemm(const PairArgs p) {
                                                          (i * nk + k) * 2048, 0));
       }
   };
-  float16v s1[2][2], s2[2][2];
-#pragma unroll
-  for (int i = 0; i < 4; i++) s1[i >> 1][i & 1] = s2[i >> 1][i & 1] = (float16v){};
-  auto step = [&](int d) __attribute__((always_inline)) {
-#pragma unroll
-    for (int g = 0; g < 3; g++)
-#pragma unroll
-      for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-          float16v &s = g == 0 ? s1[i][j] : s2[i][j];
-          s = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[d][i][g == 2], b[d][j][g == 1], s, 0, 0, 0);
-        }
-  };
   // The tile's exponents (images reach to whole 64-row blocks) and a column's
   // C where C is a row: read here, not in the epilogue, where each would be a
   // round trip of its own.
@@ -236,20 +199,8 @@ __global__ __launch_bounds__(256, 2) void k_pair_gemm(const PairArgs p) {
   if (p.c && p.c_rs == 0)
 #pragma unroll
     for (int j = 0; j < 2; j++) cb[j] = p.c[min(c0 + 32 * j + l32, p.N - 1) * p.c_cs];
-#pragma unroll
-  for (int d = 0; d < D; d++) load(d, d);
-  __syncthreads();  // exps
-  int k = 0;
-  for (; k + D <= per; k += D) {
-#pragma unroll
-    for (int d = 0; d < D; d++) {
-      step(d);
-      load(d, k + D + d);
-    }
-  }
-#pragma unroll
-  for (int d = 0; d < D; d++)
-    if (k + d < per) step(d);
+  float16v s1[2][2];
+  pair_sums(a, b, per, s1, load);
   // y = sum 2^-(ea + eb) of the 32 x 32 block (i, j) of the tile: lane
   // l holds column l % 32 and rows 8 (v / 4) + 4 (l / 32) + v % 4.  Stores
   // past M or N go past the resource and are dropped in hardware.
@@ -292,31 +243,8 @@ __global__ __launch_bounds__(256, 2) void k_pair_gemm(const PairArgs p) {
           tr0 + lr < p.M && col < p.N ? (unsigned)(lr * (int)p.ldy + l32) * 4u : 0x80000000u, 0, 0);
     }
   };
-#pragma unroll
-  for (int i = 0; i < 2; i++)
-#pragma unroll
-    for (int j = 0; j < 2; j++)
-#pragma unroll
-      for (int v = 0; v < 16; v++) s1[i][j][v] = fmaf(s2[i][j][v], 1.f / 2048.f, s1[i][j][v]);
-#pragma unroll
-  for (int q = 0; q < 4; q++)
-#pragma unroll
-    for (int v = 0; v < 4; v++) {
-      const float16v &s = s1[q >> 1][q & 1];
-      part[wave][q][v][lane] = (float4v){s[4 * v], s[4 * v + 1], s[4 * v + 2], s[4 * v + 3]};
-    }
-  __syncthreads();
-  // Wave q finishes block q.
-  float16v sum;
-#pragma unroll
-  for (int v = 0; v < 4; v++) {
-    float4v x = part[0][wave][v][lane];
-#pragma unroll
-    for (int w = 1; w < KW; w++) x += part[w][wave][v][lane];
-#pragma unroll
-    for (int e = 0; e < 4; e++) sum[4 * v + e] = x[e];
-  }
-  finish(sum, wave >> 1, wave & 1);
+  // (The barrier of the sum also publishes exps.)
+  finish(pair_reduce(part, wave, lane, s1), wave >> 1, wave & 1);
 }
 
 }  // namespace

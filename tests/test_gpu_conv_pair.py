@@ -1,0 +1,111 @@
+"""fp32 Conv on fp16 digit pairs against float64, at the edges of its 16-channel
+blocks, 64 x 64 tiles and padded windows, over 1-D to 3-D geometries, with Inf
+and NaN, and without its workspace (the fp32 MFMA kernel)."""
+import numpy as np
+import pytest
+import torch
+import torch.nn.functional as F
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from onnx_runtime_dart_amd import ops as _ops
+    return _ops
+
+
+def reference(x, w, b, stride, pads, dil):
+    """(result, its sum of magnitudes) in float64; pads as ONNX lists them."""
+    r = x.ndim - 2
+    conv = (F.conv1d, F.conv2d, F.conv3d)[r - 1]
+    pad = [q for d in range(r - 1, -1, -1) for q in (pads[d], pads[r + d])]
+    xt, wt, bt = (torch.from_numpy(t.astype(np.float64)) for t in (x, w, b))
+    y = conv(F.pad(xt, pad), wt, bt, stride=stride, dilation=dil).numpy()
+    m = conv(F.pad(xt.abs(), pad), wt.abs(), bt.abs(), stride=stride, dilation=dil).numpy()
+    return y, m
+
+
+def check(y, x, w, b, stride, pads, dil):
+    """Two digits leave 2^-23 of an operand, lo lo' 2^-24 of a product, and
+    each of the K / 16 additions (and the last few) 2^-23 of the sum."""
+    want, size = reference(x, w, b, stride, pads, dil)
+    k = np.prod(w.shape[1:])
+    steps = -(-w.shape[1] // 16) * np.prod(w.shape[2:])
+    assert k >= 256
+    assert y.shape == want.shape
+    assert (np.abs(y - want) <= (steps + 12) * 2.0**-23 * size).all()
+
+
+CASES = [  # x, w, stride, pads, dilation
+    ((2, 256, 9), (65, 256, 1), (1,), (0, 0), (1,)),
+    ((3, 100, 40), (5, 100, 7), (3,), (2, 5), (2,)),
+    ((2, 33, 11, 13), (70, 33, 3, 3), (1, 1), (1, 1, 1, 1), (1, 1)),
+    ((1, 17, 9, 30), (63, 17, 4, 5), (2, 3), (0, 3, 2, 1), (1, 2)),
+    ((5, 256, 8, 8), (64, 256, 1, 1), (2, 2), (0, 0, 0, 0), (1, 1)),
+    ((1, 16, 3, 3), (1, 16, 5, 5), (1, 1), (2, 2, 2, 2), (1, 1)),
+    ((2, 31, 5, 6, 7), (66, 31, 3, 2, 3), (2, 1, 1), (1, 0, 2, 1, 1, 0), (1, 2, 1)),
+    ((9, 272, 7, 7), (130, 272, 3, 3), (1, 1), (1, 1, 1, 1), (1, 1)),
+]
+
+
+def draw(case, seed=0):
+    rng = np.random.default_rng(seed)
+    xs, ws = case[:2]
+    return (rng.standard_normal(xs).astype(np.float32), rng.standard_normal(ws).astype(np.float32),
+            rng.standard_normal(ws[0]).astype(np.float32))
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "x".join(map(str, c[0] + c[1])))
+def test_geometries(ops, case):
+    x, w, b = draw(case)
+    # One image of another size: every image has its own exponent.
+    x[0] *= 2.0**40
+    y = ops.op_conv(x, w, b, strides=list(case[2]), pads=list(case[3]), dilations=list(case[4]))
+    check(y, x, w, b, *case[2:])
+
+
+def test_inf_and_nan(ops):
+    # An Inf or NaN reaches the outputs whose window holds it; other images
+    # and channels are those without it, and the rest of its image is redone
+    # on fp32 products.
+    case = CASES[7]
+    x, w, b = draw(case, 1)
+    args = dict(strides=list(case[2]), pads=list(case[3]), dilations=list(case[4]))
+    clean = ops.op_conv(x, w, b, **args)
+    z = x.copy()
+    z[4, 100, 3, 2], z[7, 5, 6, 6] = np.inf, np.nan
+    y = ops.op_conv(z, w, b, **args)
+    others = [0, 1, 2, 3, 5, 6, 8]
+    np.testing.assert_array_equal(y[others], clean[others])
+    hit = np.zeros((7, 7), bool)
+    hit[2:5, 1:4] = True
+    np.testing.assert_array_equal(np.isinf(y[4]), np.broadcast_to(hit, y[4].shape))
+    want, size = reference(x, w, b, *case[2:])
+    assert (np.abs(y[4] - want[4]) <= 2448 * 2.0**-24 * size[4])[:, ~hit].all()
+    np.testing.assert_array_equal(np.isnan(y[7]).any(0),
+                                  np.logical_and.outer(np.arange(7) > 4, np.arange(7) > 4))
+    v = w.copy()
+    v[65, 0, 1, 1] = np.inf
+    y = ops.op_conv(x, v, b, **args)
+    rest = np.setdiff1d(np.arange(130), [65])
+    np.testing.assert_array_equal(y[:, rest], clean[:, rest])
+    np.testing.assert_array_equal(y[:, 65], np.sign(x[:, 0]) * np.float32(np.inf))
+
+
+def test_without_workspace(ops):
+    case = CASES[2]
+    x, w, b = draw(case, 2)
+    ctx = ops.default_context()
+    bufs = [ops.DeviceBuffer.from_array(t) for t in (x, w, b)]
+    y = ops.DeviceBuffer(2 * 70 * 11 * 13 * 4)
+    ctx.set_control(None, max_bytes=4096)
+    try:
+        ops.conv_f32_dev(bufs[0].ptr, x.shape, bufs[1].ptr, w.shape, y.ptr, bufs[2].ptr,
+                         strides=[1, 1], pads=[1] * 4, ctx=ctx)
+    finally:
+        ctx.set_control(None, max_bytes=-1)
+    want, size = reference(x, w, b, *case[2:])
+    assert (np.abs(y.to_array(want.shape, np.float32) - want) <= 297 * 2.0**-23 * size).all()
+    for d in bufs + [y]:
+        d.free()
