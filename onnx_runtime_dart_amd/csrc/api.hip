@@ -2408,11 +2408,6 @@ mg_status mg_group_query_attention_dev(
     return mg_fail(MG_INVALID_ARGUMENT, "GroupQueryAttention: null buffer");
   if (nq + npres == 0) return MG_OK;
   MG_TRY(mg_use_device(ctx));
-  const size_t pb = mg_attn_plan_split(ctx, &p);
-  const size_t qrot_bytes = do_rotary ? mg_align((size_t)nq * 4) : 0;
-  MG_TRY(mg_check_control(ctx, (int64_t)(qrot_bytes + pb)));
-  if (qrot_bytes + pb) MG_TRY(mg_ws_reserve(ctx, qrot_bytes + pb));
-  if (pb) p.part = reinterpret_cast<float *>(static_cast<char *>(ctx->ws) + qrot_bytes);
   g.k = k_dev;
   g.v = v_dev;
   g.past_k = past_key_dev;
@@ -2421,6 +2416,18 @@ mg_status mg_group_query_attention_dev(
   g.sin = sin_cache_dev;
   g.present_k = present_key_dev;
   g.present_v = present_value_dev;
+  p.mask = attention_bias_dev;
+  const int64_t dec = mg_gqa_dec_ws(ctx, g, p, q_dev, y_dev);
+  if (dec >= 0 && (dec == 0 || mg_ws_optional(ctx, (size_t)dec))) {
+    MG_TRY(mg_check_control(ctx, dec));
+    g.q = q_dev;
+    return mg_gqa_dec_run(ctx, g, p, static_cast<float *>(ctx->ws), y_dev);
+  }
+  const size_t pb = mg_attn_plan_split(ctx, &p);
+  const size_t qrot_bytes = do_rotary ? mg_align((size_t)nq * 4) : 0;
+  MG_TRY(mg_check_control(ctx, (int64_t)(qrot_bytes + pb)));
+  if (qrot_bytes + pb) MG_TRY(mg_ws_reserve(ctx, qrot_bytes + pb));
+  if (pb) p.part = reinterpret_cast<float *>(static_cast<char *>(ctx->ws) + qrot_bytes);
   return gqa_run(ctx, p, g, q_dev, do_rotary ? static_cast<float *>(ctx->ws) : nullptr,
                  attention_bias_dev, y_dev);
 }

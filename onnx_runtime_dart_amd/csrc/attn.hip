@@ -1133,7 +1133,283 @@ __global__ __launch_bounds__(256) void k_gqa_prep_blk(const mg_gqa_prep g, int n
             g.sin + (g.past + s) * g.half_rot, g.interleaved);
 }
 
+// ------------------------------------------------ fused decode step
+//
+// A decode step (one query per head, no bias) in one pass over the caches: a
+// workgroup takes a (batch, KV head) and a range of keys, reads the range's
+// K and V rows once, writes them to present as it goes (the new row RoPE'd),
+// rotates its group's queries itself and attends, then k_dec_merge adds the
+// ranges.  16 (head 64) or 32 (128) lanes hold one key's row, four dims
+// each, for the scores, the weights and the output alike: nothing goes
+// through LDS until the end, and a wave's 16 row loads are in flight
+// together.  Bound by memory: past read and present written once, 33.6 MB at
+// 4096 keys of 8 heads of 64.  The copy, the attention and the merge as
+// three launches (present read again, keys and values staged in LDS) took
+// 33 us there, this takes 15.5; at 32768 keys 123 against 62, the rate of a
+// large copy being 52.
+// Lane permutation within rows of 16 lanes (DPP control CTRL).
+template <int CTRL>
+__device__ inline float dpp(float x) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), CTRL, 0xF,
+                                                            0xF, true));
+}
+
+// Row loads of a wave per chunk, each of K and V (2 or 4 instead: 14.2 / 15.2
+// against 15.5 us at 4096 keys, 64 / 66 against 62 at 32768, 9.6 / 11.3 against
+// 7.1 at 64, where they need the merge).
+constexpr int kDecIt = 8;
+template <int NS, int LPR>
+__global__ __launch_bounds__(256) void k_gqa_dec(const mg_gqa_prep g, float *__restrict__ y,
+                                                 float *__restrict__ part, int S, int kc,
+                                                 float scale2) {
+  constexpr int D = 4 * LPR, RPI = 64 / LPR, IT = kDecIt, RW = IT * RPI;  // a wave's keys per chunk
+  const int lane = threadIdx.x & 63, r = lane / LPR, d = 4 * (lane % LPR);
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int nbh = (int)gridDim.x, bh = (int)blockIdx.x;
+  const int b = bh / (int)g.kv_heads, kvh = bh - b * (int)g.kv_heads;
+  const int past = (int)g.past, T = past + 1;
+  const int t_end = min(T, ((int)blockIdx.y + 1) * kc);
+  auto rsrc = [](const float *base) __attribute__((always_inline)) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(base), (short)0, 0x7ffffff0,
+                                             0x00020000);
+  };
+  const __amdgpu_buffer_rsrc_t rk = rsrc(g.past_k + (int64_t)bh * past * D),
+                               rv = rsrc(g.past_v + (int64_t)bh * past * D);
+  const __amdgpu_buffer_rsrc_t wk = rsrc(g.present_k + (int64_t)bh * T * D),
+                               wv = rsrc(g.present_v + (int64_t)bh * T * D);
+  auto ld = [](__amdgpu_buffer_rsrc_t rs, unsigned off) __attribute__((always_inline)) {
+    return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0));
+  };
+  constexpr unsigned kOob = 0x80000000u;
+  const float *cs = g.cos + (int64_t)past * g.half_rot, *sn = g.sin + (int64_t)past * g.half_rot;
+  float4 q[NS], o[NS];
+  float m[NS], l[NS];
+  const float *q0 = g.q + ((int64_t)b * g.heads + kvh * S) * D;
+#pragma unroll
+  for (int i = 0; i < NS; i++) {
+    const float *qr = q0 + (i < S ? i : 0) * D;
+    q[i] = g.rotary ? rope4(qr, d, g.half_rot, cs, sn, g.interleaved)
+                    : *reinterpret_cast<const float4 *>(qr + d);
+    o[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    m[i] = -INFINITY, l[i] = 0.f;
+  }
+  for (int tb = (int)blockIdx.y * kc; tb < t_end; tb += 4 * RW) {
+    const int t0 = tb + wave * RW + r;
+    float4 k[IT], v[IT];
+#pragma unroll
+    for (int i = 0; i < IT; i++) {
+      const int t = t0 + i * RPI;
+      const unsigned off = t < t_end && t < past ? (unsigned)(t * D + d) * 4u : kOob;
+      k[i] = ld(rk, off);
+      v[i] = ld(rv, off);
+    }
+    if (tb + 4 * RW > past) {  // uniform: the chunk may hold the new row
+      const int64_t row = ((int64_t)b * g.kv_heads + kvh) * D;
+      const float4 nk = g.rotary ? rope4(g.k + row, d, g.half_rot, cs, sn, g.interleaved)
+                                 : *reinterpret_cast<const float4 *>(g.k + row + d);
+      const float4 nv = *reinterpret_cast<const float4 *>(g.v + row + d);
+#pragma unroll
+      for (int i = 0; i < IT; i++)
+        if (t0 + i * RPI == past) k[i] = nk, v[i] = nv;
+    }
+    float x[IT][NS];
+#pragma unroll
+    for (int i = 0; i < IT; i++) {
+      const int t = t0 + i * RPI;
+      const unsigned off = t < t_end ? (unsigned)(t * D + d) * 4u : kOob;
+      typedef unsigned u4 __attribute__((ext_vector_type(4)));
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, k[i]), wk, off, 0, 0);
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v[i]), wv, off, 0, 0);
+#pragma unroll
+      for (int s = 0; s < NS; s++) {
+        float a = q[s].x * k[i].x;
+        a = fmaf(q[s].y, k[i].y, a);
+        a = fmaf(q[s].z, k[i].z, a);
+        a = fmaf(q[s].w, k[i].w, a);
+        // Sum over the row's lanes: within quads, halves of 8, of 16 (of 32).
+        a += dpp<0xB1>(a);   // quad_perm [1, 0, 3, 2]
+        a += dpp<0x4E>(a);   // quad_perm [2, 3, 0, 1]
+        a += dpp<0x141>(a);  // row_half_mirror
+        a += dpp<0x140>(a);  // row_mirror
+        if constexpr (LPR == 32) a += __shfl_xor(a, 16);
+        x[i][s] = t < t_end ? a * scale2 : -INFINITY;
+      }
+    }
+    // Online softmax per row group of lanes (merged at the end).
+#pragma unroll
+    for (int s = 0; s < NS; s++) {
+      float mn = m[s];
+#pragma unroll
+      for (int i = 0; i < IT; i++) mn = fmaxf(mn, x[i][s]);
+      const float mz = mn == -INFINITY ? 0.f : mn;  // no key yet: weights 2^-inf = 0
+      const float corr = __builtin_amdgcn_exp2f(m[s] - mz);
+      m[s] = mn;
+      l[s] *= corr;
+      o[s].x *= corr, o[s].y *= corr, o[s].z *= corr, o[s].w *= corr;
+#pragma unroll
+      for (int i = 0; i < IT; i++) {
+        const float w = __builtin_amdgcn_exp2f(x[i][s] - mz);
+        l[s] += w;
+        o[s].x = fmaf(w, v[i].x, o[s].x);
+        o[s].y = fmaf(w, v[i].y, o[s].y);
+        o[s].z = fmaf(w, v[i].z, o[s].z);
+        o[s].w = fmaf(w, v[i].w, o[s].w);
+      }
+    }
+  }
+  // The 4 RPI row groups of the workgroup, in order.
+  constexpr int NG = 4 * RPI;
+  __shared__ float gm[NG][NS], gl[NG][NS];
+  __shared__ __attribute__((aligned(16))) float go[NG][NS][D];
+  const int grp = wave * RPI + r;
+#pragma unroll
+  for (int s = 0; s < NS; s++) {
+    if (d == 0) gm[grp][s] = m[s], gl[grp][s] = l[s];
+    *reinterpret_cast<float4 *>(&go[grp][s][d]) = o[s];
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < S * D; e += 256) {
+    const int s = e / D, dv = e - s * D;
+    float M = -INFINITY;
+#pragma unroll
+    for (int u = 0; u < NG; u++) M = fmaxf(M, gm[u][s]);
+    const float mz = M == -INFINITY ? 0.f : M;
+    float num = 0.f, den = 0.f;
+#pragma unroll
+    for (int u = 0; u < NG; u++) {
+      const float w = __builtin_amdgcn_exp2f(gm[u][s] - mz);
+      num = fmaf(w, go[u][s][dv], num);
+      den = fmaf(w, gl[u][s], den);
+    }
+    const int64_t row = (int64_t)bh * S + s;
+    if (part) {
+      float *pr = part + ((int64_t)blockIdx.y * nbh * S + row) * attn_part_row(D);
+      pr[dv] = num;
+      if (dv == 0) pr[D] = M, pr[D + 1] = den;
+    } else {
+      y[row * D + dv] = M == -INFINITY ? __builtin_nanf("") : num / den;
+    }
+  }
+}
+
+// Merge of k_gqa_dec's key ranges: a workgroup per output row, 256 / (D / 4)
+// ranges at a time, every load of up to four rounds in flight together with
+// the maxima (33 ranges: 2.2-3.7 us; one wave per row with the ranges in its
+// registers took 8.0).
+template <int LPR>
+__global__ __launch_bounds__(256) void k_dec_merge(const float *__restrict__ part, int nsplit,
+                                                   int64_t rows, float *__restrict__ y) {
+  constexpr int D = 4 * LPR, PR = (int)attn_part_row(D), G = 256 / LPR, U = 4;
+  const int t = threadIdx.x, d = 4 * (t % LPR), grp = t / LPR;
+  const int64_t row = blockIdx.x, cs = rows * PR;
+  const float *p0 = part + row * PR;
+  float4 o[U];
+  float l[U], mc[U];
+#pragma unroll
+  for (int u = 0; u < U; u++) {
+    const float *pr = p0 + min(grp + G * u, nsplit - 1) * cs;
+    o[u] = *reinterpret_cast<const float4 *>(pr + d);
+    mc[u] = pr[D], l[u] = pr[D + 1];
+  }
+  float M = -INFINITY;
+  for (int c = t; c < nsplit; c += 256) M = fmaxf(M, p0[c * cs + D]);
+#pragma unroll
+  for (int w = 32; w >= 1; w >>= 1) M = fmaxf(M, __shfl_xor(M, w));
+  __shared__ float wm[4], gden[G];
+  __shared__ __attribute__((aligned(16))) float gnum[G][D];
+  if ((t & 63) == 0) wm[t >> 6] = M;
+  __syncthreads();
+  M = fmaxf(fmaxf(wm[0], wm[1]), fmaxf(wm[2], wm[3]));
+  const float mz = M == -INFINITY ? 0.f : M;
+  float4 num = make_float4(0.f, 0.f, 0.f, 0.f);
+  float den = 0.f;
+  auto add = [&](float mm, float ll, const float4 &oo) __attribute__((always_inline)) {
+    const float w = __builtin_amdgcn_exp2f(mm - mz);
+    num.x = fmaf(w, oo.x, num.x), num.y = fmaf(w, oo.y, num.y);
+    num.z = fmaf(w, oo.z, num.z), num.w = fmaf(w, oo.w, num.w);
+    den = fmaf(w, ll, den);
+  };
+#pragma unroll
+  for (int u = 0; u < U; u++)
+    if (grp + G * u < nsplit) add(mc[u], l[u], o[u]);
+  for (int c = grp + G * U; c < nsplit; c += G) {
+    const float *pr = p0 + c * cs;
+    add(pr[D], pr[D + 1], *reinterpret_cast<const float4 *>(pr + d));
+  }
+  *reinterpret_cast<float4 *>(&gnum[grp][d]) = num;
+  if (d == 0) gden[grp] = den;
+  __syncthreads();
+  if (t >= D) return;
+  float n = 0.f, dn = 0.f;
+#pragma unroll
+  for (int u = 0; u < G; u++) n += gnum[u][t], dn += gden[u];
+  y[row * D + t] = M == -INFINITY ? __builtin_nanf("") : n / dn;
+}
+
 }  // namespace
+
+// Whether a step takes the fused kernels: one query per head, no bias, heads
+// of 64 or 128 in groups of at most 8, whole aligned quads (as
+// k_gqa_prep_blk), 32-bit offsets within a cache.
+static bool gqa_dec_ok(const mg_gqa_prep &g, const mg_attn_problem &p, const float *q,
+                       const float *y) {
+  auto al = [](const void *ptr) { return reinterpret_cast<uintptr_t>(ptr) % 16 == 0; };
+  return g.seq == 1 && !p.mask && (g.hs == 64 || g.hs == 128) && p.S <= 8 && p.nbd == 2 &&
+         al(q) && al(y) && al(g.k) && al(g.v) && al(g.present_k) && al(g.present_v) &&
+         (g.past == 0 || (al(g.past_k) && al(g.past_v))) &&
+         (!g.rotary || ((g.interleaved ? g.half_rot % 2 == 0 : g.half_rot % 4 == 0) && al(g.cos) &&
+                        al(g.sin) && 2 * g.half_rot <= g.hs)) &&
+         (g.past + 1) * g.hs < ((int64_t)1 << 28) && g.batch * g.kv_heads < (1 << 24) &&
+         g.batch * g.kv_heads > 0;
+}
+
+// Keys per workgroup: whole chunks (128 keys of heads of 64, 64 of 128), about
+// four workgroups per CU, at most 512 ranges.
+static int64_t gqa_dec_range(const mg_ctx *ctx, const mg_gqa_prep &g) {
+  const int64_t ch = kDecIt * (g.hs == 64 ? 16 : 8), total = g.past + 1, nbh = g.batch * g.kv_heads;
+  const int64_t want = std::min<int64_t>(512, (4 * (int64_t)ctx->num_cus + nbh - 1) / nbh);
+  return ((total + want - 1) / want + ch - 1) / ch * ch;
+}
+
+int64_t mg_gqa_dec_ws(const mg_ctx *ctx, const mg_gqa_prep &g, const mg_attn_problem &p,
+                      const float *q, const float *y) {
+  if (!gqa_dec_ok(g, p, q, y)) return -1;
+  const int64_t kc = gqa_dec_range(ctx, g), ns = (g.past + kc) / kc;
+  return ns < 2 ? 0 : ns * g.batch * g.kv_heads * p.S * attn_part_row(g.hs) * 4;
+}
+
+mg_status mg_gqa_dec_run(mg_ctx *ctx, const mg_gqa_prep &g, const mg_attn_problem &p, float *part,
+                         float *y) {
+  const int kc = (int)gqa_dec_range(ctx, g);
+  const int nbh = (int)(g.batch * g.kv_heads), nsplit = (int)((g.past + kc) / kc);
+  const dim3 grid((unsigned)nbh, (unsigned)nsplit);
+  const float scale2 = p.scale * 1.4426950408889634f;
+  float *pt = nsplit > 1 ? part : nullptr;
+#define MG_DEC(NS, LPR)                                                                        \
+  hipLaunchKernelGGL((k_gqa_dec<NS, LPR>), grid, dim3(256), 0, ctx->stream, g, y, pt, p.S, kc, \
+                     scale2)
+#define MG_DEC_S(LPR)                \
+  do {                               \
+    if (p.S == 1) MG_DEC(1, LPR);      \
+    else if (p.S == 2) MG_DEC(2, LPR); \
+    else if (p.S <= 4) MG_DEC(4, LPR); \
+    else MG_DEC(8, LPR);               \
+  } while (0)
+  if (g.hs == 64) MG_DEC_S(16);
+  else MG_DEC_S(32);
+#undef MG_DEC_S
+#undef MG_DEC
+  MG_TRY(mg_launch_check("k_gqa_dec"));
+  if (!pt) return MG_OK;
+  const int64_t rows = (int64_t)nbh * p.S;
+  if (g.hs == 64)
+    hipLaunchKernelGGL(k_dec_merge<16>, dim3((unsigned)rows), dim3(256), 0, ctx->stream, pt,
+                       nsplit, rows, y);
+  else
+    hipLaunchKernelGGL(k_dec_merge<32>, dim3((unsigned)rows), dim3(256), 0, ctx->stream, pt,
+                       nsplit, rows, y);
+  return mg_launch_check("k_dec_merge");
+}
 
 mg_status mg_gqa_prep_run(mg_ctx *ctx, const mg_gqa_prep &g) {
   auto al = [](const void *ptr) { return reinterpret_cast<uintptr_t>(ptr) % 16 == 0; };

@@ -471,6 +471,13 @@ struct mg_gqa_prep {
   int rotary, interleaved;
 };
 mg_status mg_gqa_prep_run(mg_ctx *ctx, const mg_gqa_prep &g);
+// A decode step in one pass over the caches (k_gqa_dec): the workspace of its
+// partials, or -1 where the step does not take this route, and its launches
+// (g.q set to the query).
+int64_t mg_gqa_dec_ws(const mg_ctx *ctx, const mg_gqa_prep &g, const mg_attn_problem &p,
+                      const float *q, const float *y);
+mg_status mg_gqa_dec_run(mg_ctx *ctx, const mg_gqa_prep &g, const mg_attn_problem &p, float *part,
+                         float *y);
 
 // --------------------------------------------------------------- DQL entry
 
