@@ -1462,8 +1462,9 @@ struct NbitsPlan {
 
 // ng_total / n_total: column groups / columns of all weights launched together
 // (sibling weights sharing one input).
-NbitsPlan plan_nbits(const mg_ctx *ctx, const mg_weight *w, int64_t M, int64_t ng_total,
-                     int64_t n_total, bool imgs) {
+// wide: prefill plans that spend workspace on further K splits.
+NbitsPlan plan_nbits_ws(const mg_ctx *ctx, const mg_weight *w, int64_t M, int64_t ng_total,
+                        int64_t n_total, bool imgs, bool wide) {
   const mg_nbits_dev &d = w->nbits;
   NbitsPlan p;
   p.M = M;
@@ -1598,7 +1599,14 @@ NbitsPlan plan_nbits(const mg_ctx *ctx, const mg_weight *w, int64_t M, int64_t n
     const int64_t mt = p.mpad / rows;
     // 128-column tiles when they alone cover the chip, else 64-column tiles;
     // then split K until the grid covers it.
-    p.nt = mt * (ng_total / 2) >= target ? 4 : 2;
+    const int64_t t4 = mt * (ng_total / 2), t2 = mt * ng_total;
+    p.nt = t4 >= target ? 4 : 2;
+    // fp16 GEMM: 64-column tiles too where the fullest CU then gets less work
+    // (301 rows x 16384 columns: 384 wide tiles put two on half of the CUs,
+    // 768 narrow ones three on each: 68.8 -> 61.8 us; at equal counts the wide
+    // ones are as fast or faster, 1000 x 12000: 106.7 / 110.8).
+    if (p.path == 1 && wide && (t2 + target - 1) / target < 2 * ((t4 + target - 1) / target))
+      p.nt = 2;
     const int64_t tiles = mt * (p.nt == 4 ? ng_total / 2 : ng_total);
     int64_t ks = 1;
     while (tiles * ks * 2 <= target && d.c4 / (ks * 2) >= MG_PREFILL_MIN_KG) ks *= 2;
@@ -1616,6 +1624,12 @@ NbitsPlan plan_nbits(const mg_ctx *ctx, const mg_weight *w, int64_t M, int64_t n
       p.kwave = 1;
       ks = 1;
     }
+    // fp16 GEMM on at most three quarters of the CUs: up to three workgroups
+    // per CU from further K splits of at least 4 k groups, whose waits overlap
+    // (301 rows, 8192 -> 2048: 2 splits 66.0, 4 55.7, 8 52.3 us; 2048 -> 3072:
+    // 1 / 2 / 4 / 8 31.7 / 30.8 / 28.2 / 30.1; with 256 tiles none is faster).
+    if (p.path == 1 && wide && 4 * tiles <= 3 * target)
+      ks = std::max(ks, std::min(3 * target / tiles, d.c4 / 4));
     p.kps = (int)((d.c4 + ks - 1) / ks);
     p.ksplit = (int)((d.c4 + p.kps - 1) / p.kps);
     if (p.path == 4) {
@@ -1638,6 +1652,20 @@ NbitsPlan plan_nbits(const mg_ctx *ctx, const mg_weight *w, int64_t M, int64_t n
     p.total = mg_align((size_t)p.chunk * per_col * 4);
   }
   return p;
+}
+
+// The wide plan where its workspace is within the context's byte budget and
+// within what the allocation-free entry point has (or no larger than the
+// other plan's): no call is refused for the sake of a split.
+NbitsPlan plan_nbits(const mg_ctx *ctx, const mg_weight *w, int64_t M, int64_t ng_total,
+                     int64_t n_total, bool imgs) {
+  const NbitsPlan p = plan_nbits_ws(ctx, w, M, ng_total, n_total, imgs, true);
+  if (p.path != 1) return p;
+  const NbitsPlan q = plan_nbits_ws(ctx, w, M, ng_total, n_total, imgs, false);
+  const size_t lim = ctx->max_bytes >= 0
+                         ? std::min<size_t>(MG_NOALLOC_SCRATCH_BYTES, (size_t)ctx->max_bytes)
+                         : MG_NOALLOC_SCRATCH_BYTES;
+  return p.total <= std::max(q.total, lim) ? p : q;
 }
 
 GemvSet make_set(int n, const mg_weight *const *w, float *const *y) {
@@ -2196,6 +2224,8 @@ mg_status prefill_run(mg_ctx *ctx, int n, const mg_weight *const *w, const float
     else if (ul == 2) MG_SPLIT_LAUNCH(2);
     else if (ul == 3) MG_SPLIT_LAUNCH(3);
     else if (ul == 4) MG_SPLIT_LAUNCH(4);
+    else if (ul <= 6) MG_SPLIT_LAUNCH(6);
+    else if (ul <= 8) MG_SPLIT_LAUNCH(8);
     else MG_SPLIT_LAUNCH(0);
 #undef MG_SPLIT_LAUNCH
   }

@@ -1,0 +1,70 @@
+"""Prefill plans of the fp16 GEMM (blocks below 128): further K splits on grids
+of few tiles, 64-column tiles where wide ones would leave CUs without work, and
+the plan without them under a byte budget; against the oracle on a subset of
+columns."""
+import numpy as np
+import pytest
+
+import golden_io as G
+import oracle
+
+pytestmark = pytest.mark.gpu
+TOL = 1e-3
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from onnx_runtime_dart_amd import ops as _ops
+    return _ops
+
+
+def weight(ops, rng, k, n, bs):
+    nb = -(-k // bs)
+    b = rng.integers(0, 256, (n, nb, bs // 2), dtype=np.uint8)
+    s = rng.uniform(0.002, 0.02, (n, nb)).astype(np.float32)
+    zp = rng.integers(0, 256, (n, (nb + 1) // 2), dtype=np.uint8)
+    return (b, s, zp), ops.NBitsWeight(b, s, zp, k=k, n=n, block_size=bs)
+
+
+def check(y, a, w, k, bs):
+    n = len(w[0])
+    cols = np.unique(np.concatenate([np.arange(0, n, max(1, n // 48)), np.arange(n - 3, n)]))
+    ref = oracle.matmul_nbits(a, w[0][cols], w[1][cols], w[2][cols], k=k, n=len(cols),
+                              block_size=bs)
+    assert G.rms_error(y[:, cols], ref) <= TOL
+
+
+@pytest.mark.parametrize("m,k,n,bs", [
+    (301, 8192, 2048, 32),   # 96 tiles: 8 splits
+    (17, 32 * 67, 130, 32),  # 3 tiles, 17 k groups: splits of uneven length
+    (129, 640, 6144, 64),    # 192 tiles (three quarters of 256 CUs), 5 k groups: one split
+    (129, 1024, 6145, 64),   # 194 tiles: above the line
+    (301, 256, 16384, 32),   # 384 wide tiles: 768 narrow ones instead
+    (256, 4128, 96, 32),     # few columns, 33 k groups
+])
+def test_plans(ops, m, k, n, bs):
+    rng = np.random.default_rng(m + k + n)
+    w, h = weight(ops, rng, k, n, bs)
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    check(h(a), a, w, k, bs)
+    h.release()
+
+
+def test_plan_under_a_byte_budget(ops):
+    # 12 MiB hold the activations' split and two partials (5 MB), not eight.
+    rng = np.random.default_rng(7)
+    m, k, n, bs = 301, 4096, 2048, 32
+    w, h = weight(ops, rng, k, n, bs)
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    ad, yd = ops.DeviceBuffer.from_array(a), ops.DeviceBuffer(m * n * 4)
+    ctx = ops.default_context()
+    for budget in (-1, 12 << 20):
+        ctx.set_control(None, max_bytes=budget)
+        try:
+            h.run_dev(ad.ptr, m, yd.ptr)
+        finally:
+            ctx.set_control(None, max_bytes=-1)
+        check(yd.to_array((m, n), np.float32), a, w, k, bs)
+    for d in (ad, yd):
+        d.free()
+    h.release()
