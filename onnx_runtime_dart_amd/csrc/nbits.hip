@@ -64,17 +64,22 @@ namespace {
 // ahl[((m32 * c4n + kg) * 8 + st) * 128 + 32 h + r] holds the hi fp16 x 8 of
 // row r, k = 128 kg + 16 st + 8 h .. +7, and +64 the lo part; texp[row] = e.
 // Rows past M and k past K are zeros.  Non-finite values pass through in hi.
-// Workgroup: 4 rows, each row on one wave.  UL > 0: the row's 16-k pieces are
-// at most 64 UL, and each lane reads its UL pieces once, with all loads in
-// flight together, and keeps them in registers for the split; UL = 0 (longer
-// rows) reads the row twice.
+// Workgroup: one row, so that a few hundred rows reach every CU, neighbouring
+// rows (whose 16-byte pieces share lines) on one XCD.  Bound by the CUs' rate:
+// 301 rows of 8192 k took 16 us on 96 workgroups with a wave a row, 12.4 with
+// the row kept in registers, 15.7 on 48 of 8 rows that fill whole lines, 10.1 so.
+// UL > 0: a row has at most 256 UL 16-k pieces, and each lane reads its UL
+// pieces once, with all loads in flight together, and keeps them in registers
+// for the split; UL = 0 (longer rows) reads the row twice.
 template <int UL>
 __global__ __launch_bounds__(256) void k_af16split(
     const float *__restrict__ a, int64_t M, int64_t K, int c4n, int vec,
     uint4 *__restrict__ ahl, int *__restrict__ texp) {
   const int t = threadIdx.x;
-  const int u0 = t & 63;
-  const int64_t row = (int64_t)blockIdx.x * 4 + (t >> 6);
+  constexpr int TPR = 256;
+  const int u0 = t;
+  // (The grid is the padded rows, a multiple of 128.)
+  const int64_t row = (int64_t)(blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
   const int64_t m32 = row >> 5;
   const int r = (int)(row & 31);
   const int units = c4n * 8;  // 16-k pieces of the row
@@ -95,6 +100,10 @@ __global__ __launch_bounds__(256) void k_af16split(
   };
   auto row_exponent = [&](float mx) {
     for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+    __shared__ float wmx[4];
+    if ((t & 63) == 0) wmx[t >> 6] = mx;
+    __syncthreads();
+    mx = fmaxf(fmaxf(wmx[0], wmx[1]), fmaxf(wmx[2], wmx[3]));
     int e = 0;
     if (mx > 0.f) {
       int ex;
@@ -127,8 +136,8 @@ __global__ __launch_bounds__(256) void k_af16split(
     float v[UL][16];
 #pragma unroll
     for (int j = 0; j < UL; j++) {
-      if (u0 + 64 * j < units) {
-        load16(u0 + 64 * j, v[j]);
+      if (u0 + TPR * j < units) {
+        load16(u0 + TPR * j, v[j]);
       } else {
 #pragma unroll
         for (int i = 0; i < 16; i++) v[j][i] = 0.f;
@@ -144,9 +153,9 @@ __global__ __launch_bounds__(256) void k_af16split(
     const int e = row_exponent(mx);
 #pragma unroll
     for (int j = 0; j < UL; j++)
-      if (u0 + 64 * j < units) split(u0 + 64 * j, v[j], e);
+      if (u0 + TPR * j < units) split(u0 + TPR * j, v[j], e);
   } else {
-    for (int u = u0; u < units; u += 64) {
+    for (int u = u0; u < units; u += TPR) {
       float v[16];
       load16(u, v);
 #pragma unroll
@@ -156,7 +165,7 @@ __global__ __launch_bounds__(256) void k_af16split(
       }
     }
     const int e = row_exponent(mx);
-    for (int u = u0; u < units; u += 64) {
+    for (int u = u0; u < units; u += TPR) {
       float v[16];
       load16(u, v);
       split(u, v, e);
@@ -2216,16 +2225,13 @@ mg_status prefill_run(mg_ctx *ctx, int n, const mg_weight *const *w, const float
   float *part = p.ksplit > 1 ? reinterpret_cast<float *>(base + p.off_c) : nullptr;
   const int vec = (w0->K % 4 == 0) && (reinterpret_cast<uintptr_t>(a_dev) % 16 == 0);
   {
-    const int ul = (int)((d.c4 * 8 + 63) / 64);  // 16-k pieces per lane
-#define MG_SPLIT_LAUNCH(UL_)                                                                   \
-  hipLaunchKernelGGL((k_af16split<UL_>), dim3((unsigned)(p.mpad / 4)), dim3(256), 0, st, a_dev, \
-                     M, w0->K, (int)d.c4, vec, ahl, texp)
-    if (ul == 1) MG_SPLIT_LAUNCH(1);
-    else if (ul == 2) MG_SPLIT_LAUNCH(2);
-    else if (ul == 3) MG_SPLIT_LAUNCH(3);
-    else if (ul == 4) MG_SPLIT_LAUNCH(4);
-    else if (ul <= 6) MG_SPLIT_LAUNCH(6);
-    else if (ul <= 8) MG_SPLIT_LAUNCH(8);
+    const int pieces = (int)((d.c4 * 8 + 255) / 256);  // 16-k pieces per lane
+#define MG_SPLIT_LAUNCH(UL_)                                                                \
+  hipLaunchKernelGGL((k_af16split<UL_>), dim3((unsigned)p.mpad), dim3(256), 0, st, a_dev, M, \
+                     w0->K, (int)d.c4, vec, ahl, texp)
+    if (pieces == 1) MG_SPLIT_LAUNCH(1);
+    else if (pieces == 2) MG_SPLIT_LAUNCH(2);
+    else if (pieces <= 4) MG_SPLIT_LAUNCH(4);
     else MG_SPLIT_LAUNCH(0);
 #undef MG_SPLIT_LAUNCH
   }
