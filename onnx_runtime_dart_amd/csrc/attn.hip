@@ -111,9 +111,15 @@ __device__ __attribute__((always_inline)) void attn_tiles(const mg_attn_problem 
 #pragma unroll
     for (int j = 0; j < DVT; j++)
 #pragma unroll
-      for (int v = 0; v < 16; v++) {
-        const int dv = 32 * j + 8 * (v >> 2) + 4 * h + (v & 3);
-        if (dv < p.DV) pr[dv] = 0.f;
+      for (int g = 0; g < 4; g++) {
+        const int dv = 32 * j + 8 * g + 4 * h;
+        if ((p.DV & 3) == 0) {
+          if (dv < p.DV) *reinterpret_cast<float4 *>(pr + dv) = make_float4(0.f, 0.f, 0.f, 0.f);
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; i++)
+            if (dv + i < p.DV) pr[dv + i] = 0.f;
+        }
       }
     if (h == 0) pr[p.DV] = -INFINITY, pr[p.DV + 1] = 0.f;
     return;
@@ -375,18 +381,33 @@ __device__ __attribute__((always_inline)) void attn_tiles(const mg_attn_problem 
 
   const float l_tot = l_run + __shfl_xor(l_run, 32);
   if (!active || !qok) return;
+  // This query's outputs: a lane's registers are quads of neighbouring dims,
+  // 16-byte stores where the row allows them (64 lanes store to 64 rows: with
+  // 4-byte stores the row addresses, not the bytes, bounded the epilogue).
+  auto store = [&](float *r, bool quads, float f) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < DVT; j++)
+#pragma unroll
+      for (int g = 0; g < 4; g++) {
+        const int dv = 32 * j + 8 * g + 4 * h;
+        const float4 x = make_float4(o[j][4 * g] * f, o[j][4 * g + 1] * f, o[j][4 * g + 2] * f,
+                                     o[j][4 * g + 3] * f);
+        if (quads) {
+          if (dv < p.DV) *reinterpret_cast<float4 *>(r + dv) = x;
+        } else {
+          if (dv < p.DV) r[dv] = x.x;
+          if (dv + 1 < p.DV) r[dv + 1] = x.y;
+          if (dv + 2 < p.DV) r[dv + 2] = x.z;
+          if (dv + 3 < p.DV) r[dv + 3] = x.w;
+        }
+      }
+  };
   if (p.part) {
     // Partial of this key split: unnormalised O, the running max (log2
     // domain) and the sum, [split][batch index][query][attn_part_row(DV)].
     float *pr = p.part + (((int64_t)blockIdx.y * (gridDim.x / qtiles) + bi) * p.S + q) *
                              attn_part_row(p.DV);
-#pragma unroll
-    for (int j = 0; j < DVT; j++)
-#pragma unroll
-      for (int v = 0; v < 16; v++) {
-        const int dv = 32 * j + 8 * (v >> 2) + 4 * h + (v & 3);
-        if (dv < p.DV) pr[dv] = o[j][v];
-      }
+    store(pr, (p.DV & 3) == 0, 1.f);
     if (h == 0) pr[p.DV] = m_run, pr[p.DV + 1] = l_tot;
     return;
   }
@@ -398,13 +419,12 @@ __device__ __attribute__((always_inline)) void attn_tiles(const mg_attn_problem 
   else
     inv = 1.f / l_tot;
   float *yr = p.y + oy + (int64_t)q * p.y_rs;
+  if (p.T == 0) {
 #pragma unroll
-  for (int j = 0; j < DVT; j++)
-#pragma unroll
-    for (int v = 0; v < 16; v++) {
-      const int dv = 32 * j + 8 * (v >> 2) + 4 * h + (v & 3);
-      if (dv < p.DV) yr[dv] = p.T == 0 ? 0.f : o[j][v] * inv;
-    }
+    for (int j = 0; j < DVT; j++) o[j] = (float16v){};
+  }
+  store(yr, (p.DV & 3) == 0 && (p.y_rs & 3) == 0 && (reinterpret_cast<uintptr_t>(p.y + oy) & 15) == 0,
+        inv);
 }
 
 // Head sizes whose fragments and accumulators fit 256 registers run at two
