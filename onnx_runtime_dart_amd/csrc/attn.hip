@@ -49,6 +49,15 @@ typedef float float16v __attribute__((ext_vector_type(16)));
 // that rows start 16-byte aligned (the merge reads four outputs at a time).
 __host__ __device__ constexpr int64_t attn_part_row(int64_t dv) { return (dv + 5) & ~int64_t(3); }
 
+// Key splits that hold a key visible to query q's tile of 128 queries: with
+// causal masking the tiled kernel writes no partials past them (300 tokens, 8
+// heads of 64: 22.8 -> 21.4 us).
+__device__ inline int attn_splits(const mg_attn_problem &p, int q, int nsplit) {
+  if (!p.causal) return nsplit;
+  const int64_t last = (int64_t)(q | 127) + p.causal_off;  // last key the tile sees
+  return last < 0 ? 0 : (int)std::min<int64_t>(nsplit, last / p.kc + 1);
+}
+
 template <int DS, int DVT>
 __device__ __attribute__((always_inline)) void attn_tiles(const mg_attn_problem &p) {
   // Tiles prefetched ahead in registers: two for head size <= 32, one for the
@@ -102,26 +111,8 @@ __device__ __attribute__((always_inline)) void attn_tiles(const mg_attn_problem 
     t_loop = (int)std::min<int64_t>(t_loop, std::max<int64_t>(0, q_last + p.causal_off + 1));
   }
   if (p.part && t_loop <= t_begin) {
-    // A split past the causal limit of every query of the tile: its partial
-    // is that of no keys (zero O, max -inf, sum 0), written without loading
-    // anything (the whole workgroup leaves here).
-    if (!active || !qok) return;
-    float *pr = p.part + (((int64_t)blockIdx.y * (gridDim.x / qtiles) + bi) * p.S + q) *
-                             attn_part_row(p.DV);
-#pragma unroll
-    for (int j = 0; j < DVT; j++)
-#pragma unroll
-      for (int g = 0; g < 4; g++) {
-        const int dv = 32 * j + 8 * g + 4 * h;
-        if ((p.DV & 3) == 0) {
-          if (dv < p.DV) *reinterpret_cast<float4 *>(pr + dv) = make_float4(0.f, 0.f, 0.f, 0.f);
-        } else {
-#pragma unroll
-          for (int i = 0; i < 4; i++)
-            if (dv + i < p.DV) pr[dv + i] = 0.f;
-        }
-      }
-    if (h == 0) pr[p.DV] = -INFINITY, pr[p.DV + 1] = 0.f;
+    // A split past the causal limit of every query of the tile: the merge
+    // does not read it (attn_splits; the whole workgroup leaves here).
     return;
   }
 
@@ -688,6 +679,7 @@ __global__ __launch_bounds__(256) void k_attn_combine(const mg_attn_problem p, i
   }
   const float *p0 = p.part + row * attn_part_row(p.DV);
   const int64_t cs = nbatch * p.S * attn_part_row(p.DV);  // stride between splits
+  nsplit = attn_splits(p, q, nsplit);
   float M = -INFINITY, num = 0.f, den = 0.f;
   auto add = [&](float m, float o, float l) {
     const float w = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - M);
@@ -750,6 +742,7 @@ __global__ __launch_bounds__(256) void k_attn_combine4(const mg_attn_problem p, 
   }
   const float *p0 = p.part + row * attn_part_row(p.DV);
   const int64_t cs = nbatch * p.S * attn_part_row(p.DV);
+  nsplit = attn_splits(p, q, nsplit);
   float M = -INFINITY;
   float num[4] = {0.f, 0.f, 0.f, 0.f}, den = 0.f;
   auto add = [&](float m, const float4 &o, float l) {
@@ -817,6 +810,7 @@ __global__ __launch_bounds__(256) void k_attn_combine_w(const mg_attn_problem p,
   const float *p0 = p.part + row * attn_part_row(p.DV);
   const int64_t cs = nbatch * p.S * attn_part_row(p.DV);
   const int DV = (int)p.DV;
+  nsplit = attn_splits(p, q, nsplit);
   const float mc = lane < nsplit ? p0[lane * cs + DV] : -INFINITY;
   const float lc = lane < nsplit ? p0[lane * cs + DV + 1] : 0.f;
   float o[DPL][64];
