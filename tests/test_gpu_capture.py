@@ -1,0 +1,106 @@
+"""Ops with an optional workspace under HIP graph capture: replays give the
+eager results, also after the workspace has grown past the captured one, and a
+Gemm captured without any workspace runs the kernel that needs none."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from onnx_runtime_dart_amd import ops as _ops
+    return _ops
+
+
+class Hip:
+    """The HIP runtime that the library itself has loaded."""
+
+    def __init__(self):
+        with open("/proc/self/maps") as f:
+            path = next(line.split()[-1] for line in f if "libamdhip64" in line)
+        self.lib = C.CDLL(path)
+
+    def __getattr__(self, name):
+        def call(*args):
+            rc = getattr(self.lib, name)(*args)
+            assert rc == 0, (name, rc)
+        return call
+
+
+SHAPES = dict(a=(100, 96), x=(2, 40, 9, 9), w=(24, 40, 3, 3), q=(1, 1, 256), k=(1, 1, 128),
+              v=(1, 1, 128), pk=(1, 2, 300, 64), pv=(1, 2, 300, 64))
+OUTPUTS = dict(gemm=(100, 70), conv=(2, 24, 9, 9), gqa=(1, 1, 256), ko=(1, 2, 301, 64),
+               vo=(1, 2, 301, 64))
+
+
+def run(ops, ctx, d, fw, gemm_only):
+    fw.gemm_dev(d["a"].ptr, 100, d["gemm"].ptr)
+    if gemm_only:
+        return
+    ops.conv_f32_dev(d["x"].ptr, SHAPES["x"], d["w"].ptr, SHAPES["w"], d["conv"].ptr,
+                     strides=[1, 1], pads=[1] * 4, ctx=ctx)
+    ops.group_query_attention_dev(d["q"].ptr, d["k"].ptr, d["v"].ptr, 1, 1, 256, 4, 2,
+                                  d["gqa"].ptr, d["ko"].ptr, d["vo"].ptr, past_key_ptr=d["pk"].ptr,
+                                  past_value_ptr=d["pv"].ptr, past_len=300, ctx=ctx)
+
+
+@pytest.mark.parametrize("warm", [True, False])
+def test_graph_replays(ops, warm):
+    rng = np.random.default_rng(1)
+    ctx = ops.Context()
+    hip = Hip()
+    stream, graph, exe = C.c_void_p(), C.c_void_p(), C.c_void_p()
+    hip.hipStreamCreate(C.byref(stream))
+    ctx.set_stream(stream.value)
+    fw = ops.F32Weight(rng.standard_normal((70, 96)).astype(np.float32), trans_b=True, ctx=ctx)
+    big = ops.F32Weight(rng.standard_normal((64, 1024)).astype(np.float32), trans_b=True, ctx=ctx)
+    d = {key: ops.DeviceBuffer(4 * int(np.prod(s))) for key, s in {**SHAPES, **OUTPUTS}.items()}
+
+    def fill(names):
+        for key in names:
+            s = SHAPES.get(key) or OUTPUTS[key]
+            h = rng.standard_normal(s).astype(np.float32)
+            hip.hipMemcpy(C.c_void_p(d[key].ptr), h.ctypes.data_as(C.c_void_p),
+                          C.c_size_t(h.nbytes), 1)
+
+    def results():
+        hip.hipStreamSynchronize(stream)
+        names = OUTPUTS if warm else ["gemm"]
+        return {key: d[key].to_array(OUTPUTS[key], np.float32) for key in names}
+
+    fill(SHAPES)
+    if warm:
+        run(ops, ctx, d, fw, False)
+        hip.hipStreamSynchronize(stream)
+    hip.hipStreamBeginCapture(stream, 0)
+    run(ops, ctx, d, fw, not warm)
+    hip.hipStreamEndCapture(stream, C.byref(graph))
+    hip.hipGraphInstantiate(C.byref(exe), graph, None, None, C.c_size_t(0))
+    for step in (1, 2, 3):
+        fill(list(SHAPES) + list(OUTPUTS))
+        hip.hipGraphLaunch(exe, stream)
+        got = results()
+        fill(OUTPUTS)
+        run(ops, ctx, d, fw, not warm)
+        for key, want in results().items():
+            if warm:
+                np.testing.assert_array_equal(got[key], want)
+            else:  # the graph holds the fp32 kernel: sums of 96 products, 2^-17 of ~40
+                np.testing.assert_allclose(got[key], want, rtol=0, atol=1e-4)
+        # A workspace larger than the graph's, other data in it.
+        a, z = ops.DeviceBuffer(4096 * step * 4096), ops.DeviceBuffer(4096 * step * 256)
+        big.gemm_dev(a.ptr, 4096 * step, z.ptr)
+        hip.hipStreamSynchronize(stream)
+        a.free()
+        z.free()
+    hip.hipGraphExecDestroy(exe)
+    hip.hipGraphDestroy(graph)
+    for b in d.values():
+        b.free()
+    fw.release()
+    big.release()
+    ctx.close()
+    hip.hipStreamDestroy(stream)

@@ -3,8 +3,6 @@ blocks, 64 x 64 tiles and padded windows, over 1-D to 3-D geometries, with Inf
 and NaN, and without its workspace (the fp32 MFMA kernel)."""
 import numpy as np
 import pytest
-import torch
-import torch.nn.functional as F
 
 pytestmark = pytest.mark.gpu
 
@@ -15,15 +13,24 @@ def ops():
     return _ops
 
 
+def conv64(x, w, stride, pads, dil):
+    r = x.ndim - 2
+    x = np.pad(x, [(0, 0), (0, 0)] + [(pads[d], pads[r + d]) for d in range(r)])
+    out = [(x.shape[2 + d] - (w.shape[2 + d] - 1) * dil[d] - 1) // stride[d] + 1 for d in range(r)]
+    y = 0.0
+    for tap in np.ndindex(*w.shape[2:]):
+        at = tuple(slice(tap[d] * dil[d], tap[d] * dil[d] + (out[d] - 1) * stride[d] + 1, stride[d])
+                   for d in range(r))
+        y = y + np.moveaxis(np.tensordot(x[(..., *at)], w[(..., *tap)], ((1,), (1,))), -1, 1)
+    return y
+
+
 def reference(x, w, b, stride, pads, dil):
     """(result, its sum of magnitudes) in float64; pads as ONNX lists them."""
-    r = x.ndim - 2
-    conv = (F.conv1d, F.conv2d, F.conv3d)[r - 1]
-    pad = [q for d in range(r - 1, -1, -1) for q in (pads[d], pads[r + d])]
-    xt, wt, bt = (torch.from_numpy(t.astype(np.float64)) for t in (x, w, b))
-    y = conv(F.pad(xt, pad), wt, bt, stride=stride, dilation=dil).numpy()
-    m = conv(F.pad(xt.abs(), pad), wt.abs(), bt.abs(), stride=stride, dilation=dil).numpy()
-    return y, m
+    x, w = x.astype(np.float64), w.astype(np.float64)
+    b = b.astype(np.float64).reshape((1, -1) + (1,) * (x.ndim - 2))
+    return (conv64(x, w, stride, pads, dil) + b,
+            conv64(np.abs(x), np.abs(w), stride, pads, dil) + np.abs(b))
 
 
 def check(y, x, w, b, stride, pads, dil):
