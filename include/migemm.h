@@ -386,16 +386,21 @@ mg_status mg_gemm_f32(mg_ctx *ctx, const float *a, const int64_t *a_shape,
 
 /* Uploads an fp32 B given as stored ([rows, cols]); with trans_b the operand
  * is B^T, i.e. K = cols, N = rows (the transB prepack of
- * lib/src/onnx_graph.dart:2159-2161 done once on upload). */
+ * lib/src/onnx_graph.dart:2159-2161 done once on upload).  Beside the fp32
+ * values the weight keeps their fp16 digit pairs (4 more bytes per element,
+ * counted by mg_weight_info; left out where the device has no room). */
 mg_status mg_weight_f32_create(mg_ctx *ctx, const float *b, int64_t rows,
                                int64_t cols, int32_t trans_b, mg_weight **out);
 /* y[rows, N] = alpha * a[rows, K] . W + beta * C, C as in mg_gemm_f32 (may be
  * NULL).  With alpha = 1, beta = 0, C = NULL this is MatMul against an
  * initializer, including the shared-weight batch collapse
- * (lib/src/onnx_ops.dart:1728-1735).  With K >= 1024 and rows <= 8192 the
- * product is split over K: the call then takes up to 64 MiB of the
- * context's workspace for the partial sums (wider weights run in column
- * chunks; counted against the byte budget), also with device pointers. */
+ * (lib/src/onnx_ops.dart:1728-1735).  The call takes up to 64 MiB of the
+ * context's workspace for the digit pairs of a (longer ones run in row
+ * chunks), also with device pointers.  Where the byte budget does not allow
+ * them, or the stream is capturing and the workspace is smaller, it runs on
+ * fp32 products instead: those need none, or with K >= 1024 and rows <= 8192
+ * up to 64 MiB for partial sums of a K split (wider weights in column chunks;
+ * counted against the byte budget). */
 mg_status mg_gemm_f32_w(mg_ctx *ctx, const float *a, int64_t rows, int64_t K,
                         const mg_weight *w, float alpha, float beta,
                         const float *c, const int64_t *c_shape, int32_t c_rank,
