@@ -1159,8 +1159,16 @@ __global__ __launch_bounds__(256) void k_gqa_prep_blk(const mg_gqa_prep g, int n
 // together.  Bound by memory: past read and present written once, 33.6 MB at
 // 4096 keys of 8 heads of 64.  The copy, the attention and the merge as
 // three launches (present read again, keys and values staged in LDS) took
-// 33 us there, this takes 15.5; at 32768 keys 123 against 62, the rate of a
+// 33 us there, this takes 13.3; at 32768 keys 123 against 51, the rate of a
 // large copy being 52.
+// Present is stored non-temporally: it is next read a whole step later, after
+// every other layer's caches and weights, so it need not displace them (15.5 ->
+// 13.3 us at 4096 keys, 62 -> 51 at 32768).  Steps whose past is the step
+// before's present: 16 layers of 4096 keys 13.5 -> 12.0 a layer, 16 of 8000 by
+// 2 heads of 128 16.3 -> 14.8, 4 of 16000 35.1 -> 33.4, 8 of 32768 60.1 -> 59.8;
+// only one layer alone, its caches still in the last-level cache, loses (16000
+// keys 27 -> 33).  Non-temporal loads of past as well: 32768 keys 58.  The first
+// rows loaded ahead of the queries' rotation: 15.6 -> 16.3 (plain stores).
 // Lane permutation within rows of 16 lanes (DPP control CTRL).
 template <int CTRL>
 __device__ inline float dpp(float x) {
@@ -1170,7 +1178,7 @@ __device__ inline float dpp(float x) {
 
 // Row loads of a wave per chunk, each of K and V (2 or 4 instead: 14.2 / 15.2
 // against 15.5 us at 4096 keys, 64 / 66 against 62 at 32768, 9.6 / 11.3 against
-// 7.1 at 64, where they need the merge).
+// 7.1 at 64, where they need the merge; with plain stores).
 constexpr int kDecIt = 8;
 template <int NS, int LPR>
 __global__ __launch_bounds__(256) void k_gqa_dec(const mg_gqa_prep g, float *__restrict__ y,
@@ -1232,8 +1240,9 @@ __global__ __launch_bounds__(256) void k_gqa_dec(const mg_gqa_prep g, float *__r
       const int t = t0 + i * RPI;
       const unsigned off = t < t_end ? (unsigned)(t * D + d) * 4u : kOob;
       typedef unsigned u4 __attribute__((ext_vector_type(4)));
-      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, k[i]), wk, off, 0, 0);
-      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v[i]), wv, off, 0, 0);
+      constexpr int kNt = 2;  // non-temporal
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, k[i]), wk, off, 0, kNt);
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v[i]), wv, off, 0, kNt);
 #pragma unroll
       for (int s = 0; s < NS; s++) {
         float a = q[s].x * k[i].x;
