@@ -387,8 +387,10 @@ mg_status mg_gemm_f32(mg_ctx *ctx, const float *a, const int64_t *a_shape,
 /* Uploads an fp32 B given as stored ([rows, cols]); with trans_b the operand
  * is B^T, i.e. K = cols, N = rows (the transB prepack of
  * lib/src/onnx_graph.dart:2159-2161 done once on upload).  Beside the fp32
- * values the weight keeps their fp16 digit pairs (4 more bytes per element,
- * counted by mg_weight_info; left out where the device has no room). */
+ * values the weight keeps their fp16 digit pairs (4 more bytes per element with
+ * N padded to 64 columns and K to 64, counted by mg_weight_info).  They are left
+ * out for K > 2^18 - 64 or N >= 2^22, where the padding makes them more than
+ * twice the weight plus a MiB, and where the device has no room. */
 mg_status mg_weight_f32_create(mg_ctx *ctx, const float *b, int64_t rows,
                                int64_t cols, int32_t trans_b, mg_weight **out);
 /* y[rows, N] = alpha * a[rows, K] . W + beta * C, C as in mg_gemm_f32 (may be

@@ -603,9 +603,9 @@ mg_status mg_weight_f32_create(mg_ctx *ctx, const float *b, int64_t rows, int64_
     delete w;
     return mg_fail(MG_DEVICE_ERROR, "mg_weight_f32_create: upload failed");
   }
-  // Its pair images; a weight without them (no memory left) runs on the fp32
+  // Its pair images; a weight without them (or no memory left) runs on the fp32
   // MFMA kernel.
-  if (bytes && N < MG_PAIR_MAX_N) {
+  if (mg_pair_keeps(N, K)) {
     const size_t pb = mg_pair_bytes(N, K);
     if (hipMalloc(&w->f32.pair, pb) != hipSuccess) {
       w->f32.pair = nullptr;
@@ -1387,7 +1387,7 @@ mg_status gemm_w(mg_ctx *ctx, const float *a, bool a_dev_ptr, int64_t rows, int6
   // On pair images where the weight has them and the images of A (row chunks
   // of at most 64 MiB) can be had; else on the fp32 MFMA kernel, which needs
   // less workspace or none.
-  const int64_t chunk = std::max<int64_t>(64, ((64ll << 20) / (int64_t)mg_pair_bytes(64, K)) * 64);
+  const int64_t chunk = MG_PAIR_CHUNK_BYTES / (int64_t)mg_pair_bytes(64, K) * 64;
   const size_t pb = mg_align(mg_pair_bytes(std::min(rows, chunk), K));
   const bool pair = w->f32.pair && mg_ws_optional(ctx, s.off + pb);
   q.kspl = pair ? 1 : mg_f32_ksplit(rows, K, 1);

@@ -340,8 +340,10 @@ bool mg_f32_xcd_cut(int64_t ny, int64_t nx, int *pr, int *pc, int64_t *per);
 // Pair images (fp16 hi and lo digits in MFMA order and row exponents, see
 // pair.hip) of an fp32 matrix of R rows of K contiguous elements, and y =
 // alpha A . B^T + beta C of one batch on the images of A [M, K] and B [N, K].
-constexpr int64_t MG_PAIR_MAX_N = 1 << 22;  // 32-bit offsets within an output tile
 size_t mg_pair_bytes(int64_t R, int64_t K);
+// Whether a weight [N, K] keeps pair images.
+bool mg_pair_keeps(int64_t N, int64_t K);
+constexpr int64_t MG_PAIR_CHUNK_BYTES = 64 << 20;  // of A's images per round of launches
 mg_status mg_pair_split(mg_ctx *ctx, const float *x_dev, int64_t R, int64_t K, void *img);
 mg_status mg_pair_run(mg_ctx *ctx, const mg_f32_problem &p, const float *a_dev,
                       const void *a_img, const float *b_dev, const void *b_img, float *y_dev);

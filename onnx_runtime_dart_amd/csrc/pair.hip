@@ -258,6 +258,17 @@ size_t mg_pair_bytes(int64_t R, int64_t K) {
   return mg_align((size_t)(r * nk * 64)) + mg_align((size_t)r * 4);
 }
 
+// N: 32-bit offsets within an output tile.  K: the images of 64 rows of A, the
+// least that a call takes, within a chunk, which is at most 2^18 - 64 (the
+// fragments' 32-bit offsets would reach 2^23).  And no more than twice the
+// weight's own bytes (N >= 32 always), or a MiB, go into the images, whose rows are
+// padded to 64: a 1 x 2^20 weight of 4 MiB would take 256.
+bool mg_pair_keeps(int64_t N, int64_t K) {
+  return N > 0 && K > 0 && N < ((int64_t)1 << 22) && K < ((int64_t)1 << 18) &&
+         (int64_t)mg_pair_bytes(64, K) <= MG_PAIR_CHUNK_BYTES &&
+         (int64_t)mg_pair_bytes(N, K) <= 8 * N * K + (1 << 20);
+}
+
 mg_status mg_pair_split(mg_ctx *ctx, const float *x_dev, int64_t R, int64_t K, void *img) {
   const int64_t rp = (R + 63) / 64 * 64;
   const int nk = (int)mg_pair_steps(K);

@@ -105,3 +105,24 @@ def test_without_workspace(ops):
     for b in (ad, yd):
         b.free()
     fw.release()
+
+
+def test_long_k(ops):
+    # Above the K of pair images (32-bit fragment offsets, one chunk of A):
+    # whole numbers whose sums are exact.
+    rng = np.random.default_rng(6)
+    for m, k, n in ((33, (1 << 23) + 40, 1), (65, (1 << 18) - 64, 40), (65, (1 << 18) - 63, 40)):
+        a = rng.integers(-1, 2, (m, k), dtype=np.int8).astype(np.float32)
+        w = rng.integers(-1, 2, (n, k), dtype=np.int8).astype(np.float32)
+        fw = ops.F32Weight(w, trans_b=True)
+        y = fw.gemm(a)
+        fw.release()
+        np.testing.assert_array_equal(y, a @ w.T)
+
+
+def test_image_bytes(ops):
+    # Images are bounded by the weight's size, whatever their padding.
+    for n, k in ((1, 1 << 20), (1, 4), (7, 5000), (32, 8192), (100, 300), (40, 1 << 18)):
+        fw = ops.F32Weight(np.zeros((n, k), np.float32), trans_b=True)
+        assert 4 * n * k <= fw.info()[2] <= 12 * n * k + (1 << 20)
+        fw.release()
