@@ -396,7 +396,12 @@ mg_status mg_weight_f32_create(mg_ctx *ctx, const float *b, int64_t rows,
 /* y[rows, N] = alpha * a[rows, K] . W + beta * C, C as in mg_gemm_f32 (may be
  * NULL).  With alpha = 1, beta = 0, C = NULL this is MatMul against an
  * initializer, including the shared-weight batch collapse
- * (lib/src/onnx_ops.dart:1728-1735).  The call takes up to 64 MiB of the
+ * (lib/src/onnx_ops.dart:1728-1735).  Where the weight has digit pairs, the
+ * products are formed from them: every output is within 2^-21 of its sum of
+ * |a| |b|, beside the rounding of the fp32 sums (closer than fp32 products on
+ * ordinary data, whose sums round more often; outputs that need more, and those
+ * of rows and columns with Inf or NaN, are formed from the fp32 operands).  The
+ * call then takes up to 64 MiB of the
  * context's workspace for the digit pairs of a (longer ones run in row
  * chunks), also with device pointers.  Where the byte budget does not allow
  * them, or the stream is capturing and the workspace is smaller, it runs on
@@ -500,7 +505,13 @@ mg_status mg_group_query_attention_dev(
  * dilations NULL (all 1) or [nd]; pads NULL (all 0) or [2 nd] (all begins,
  * then all ends); auto_pad 0 NOTSET, 1 SAME_UPPER, 2 SAME_LOWER, 3 VALID,
  * resolved as the reference's _resolvePads (lib/src/onnx_nn_ops.dart:38-87).
- * y [N, M, out...] from mg_conv_output_shape (x_rank values). */
+ * y [N, M, out...] from mg_conv_output_shape (x_rank values).
+ * Long sums of one group (C * taps of 256 and more, see conv_pair.hip) are
+ * formed from fp16 digit pairs as in mg_gemm_f32_w, to the same bound.  Such a
+ * call takes context workspace for the digits, also with device pointers: 4
+ * bytes per element of the filters and of the padded inputs of up to 64 MiB of
+ * images at a time (at least one).  Without it (byte budget, stream capture) it
+ * runs on fp32 products. */
 mg_status mg_conv_output_shape(const int64_t *x_shape, int32_t x_rank,
                                const int64_t *w_shape, const int64_t *strides,
                                const int64_t *pads, const int64_t *dilations,

@@ -9,7 +9,8 @@
 //     with step = block * taps + tap, and the largest magnitude of each chunk
 //     of each image;
 //   * k_conv_pair_x: the input as [image][block][hi|lo][position][16] with the
-//     padding written out as zeros, a position being one of the padded window.
+//     padding written out as zeros, a position being one of the padded window,
+//     and the number of small elements of each image (pair_common.h).
 // So a step's operand of 32 consecutive output positions is 32-byte pieces
 // at the positions' window origins (one 32-bit offset per lane, the same in
 // every step) plus the step's own offset, a scalar: the products' loop has
@@ -24,6 +25,10 @@ namespace {
 
 constexpr int kMaxChunks = 64;  // chunk maxima per image (one per lane of a wave)
 
+// Ints between the counters that workgroups add to: a line each (32 images'
+// counters in one line, added to by every wave: 15 us).
+constexpr int kCountStride = 64;
+
 struct ConvPair {
   const float *x, *w, *bias;
   float *y;
@@ -32,7 +37,8 @@ struct ConvPair {
   int in_sp, out_sp, win_sp;
   int chunks, chunk;              // maxima chunks of an image, elements of each
   uint4 *wi, *xi;                 // images of the filters and of the input
-  int *we, *xe;                   // their exponents
+  int *we, *xe;                   // their words (pair_word; xe without the count)
+  int *xn;                        // small elements of image i at i * kCountStride
   unsigned *part;                 // [n][chunks] largest magnitudes (bits)
   int nx, pr, pc;                 // tile grid and its XCD cut
 };
@@ -49,25 +55,34 @@ __global__ __launch_bounds__(256) void k_conv_pair_prep(const ConvPair p) {
   const float *src = filt ? p.w + (int64_t)m * K : p.x + img * xn + (int64_t)ch * p.chunk;
   const int len = filt ? (m < p.m ? K : 0)
                        : (int)std::min<int64_t>(p.chunk, xn - (int64_t)ch * p.chunk);
-  unsigned mx = 0;
+  unsigned mx = 0, mn = ~0u;
   for (int i = t; i < len; i += 8 * 256) {
     float v[8];
 #pragma unroll
     for (int u = 0; u < 8; u++) v[u] = src[min(i + 256 * u, len - 1)];
 #pragma unroll
-    for (int u = 0; u < 8; u++) mx = max(mx, __builtin_bit_cast(unsigned, v[u]) & 0x7fffffffu);
+    for (int u = 0; u < 8; u++) {
+      mx = max(mx, __builtin_bit_cast(unsigned, v[u]) & 0x7fffffffu);
+      mn = min(mn, pair_bits1(v[u]));
+    }
   }
-  for (int o = 32; o > 0; o >>= 1) mx = max(mx, (unsigned)__shfl_xor((int)mx, o));
-  __shared__ unsigned wmx[4];
-  if ((t & 63) == 0) wmx[t >> 6] = mx;
+  for (int o = 32; o > 0; o >>= 1) {
+    mx = max(mx, (unsigned)__shfl_xor((int)mx, o));
+    mn = min(mn, (unsigned)__shfl_xor((int)mn, o));
+  }
+  __shared__ unsigned wmx[4], wmn[4];
+  if ((t & 63) == 0) wmx[t >> 6] = mx, wmn[t >> 6] = mn;
   __syncthreads();
   mx = max(max(wmx[0], wmx[1]), max(wmx[2], wmx[3]));
+  mn = min(min(wmn[0], wmn[1]), min(wmn[2], wmn[3]));
   if (!filt) {
     if (t == 0) p.part[q] = mx;
+    if (t == 0 && ch == 0) p.xn[img * kCountStride] = 0;
     return;
   }
   const int e = pair_exponent(mx);
-  if (t == 0) p.we[m] = e;
+  const unsigned below = pair_small_below(e);
+  int small = 0;
   // Octet o: channels 8 c8 .. +7 of tap r, then the padding steps' zeros.
   const int real = p.cb * p.taps;
   for (int o = t; o < 2 * p.ns; o += 256) {
@@ -77,6 +92,9 @@ __global__ __launch_bounds__(256) void k_conv_pair_prep(const ConvPair p) {
 #pragma unroll
       for (int j = 0; j < 8; j++)
         if (8 * c8 + j < p.c) v[j] = src[(8 * c8 + j) * p.taps + r];
+    if (mn < below)  // uniform
+#pragma unroll
+      for (int j = 0; j < 8; j++) small += pair_bits1(v[j]) < below;
     half8 hi, lo;
     pair_split8(v, e, &hi, &lo);
     const int s = o < 2 * real ? (c8 >> 1) * p.taps + r : o >> 1, h = o < 2 * real ? c8 & 1 : o & 1;
@@ -84,6 +102,14 @@ __global__ __launch_bounds__(256) void k_conv_pair_prep(const ConvPair p) {
     d[0] = __builtin_bit_cast(uint4, hi);
     d[64] = __builtin_bit_cast(uint4, lo);
   }
+  if (mn < below) {
+    for (int o = 32; o > 0; o >>= 1) small += __shfl_xor(small, o);
+    __shared__ int wsm[4];
+    if ((t & 63) == 0) wsm[t >> 6] = small;
+    __syncthreads();
+    small = wsm[0] + wsm[1] + wsm[2] + wsm[3];
+  }
+  if (t == 0) p.we[m] = pair_word(e, mx, small);
 }
 
 // Thread = one position of the padded window, 16 channels (grid: positions,
@@ -104,14 +130,25 @@ __global__ __launch_bounds__(256) void k_conv_pair_x(const ConvPair p) {
   unsigned mx = lane < p.chunks ? p.part[img * p.chunks + lane] : 0;
   for (int o = 32; o > 0; o >>= 1) mx = max(mx, (unsigned)__shfl_xor((int)mx, o));
   const int e = pair_exponent(mx);
-  if (pos == 0 && cb == 0) p.xe[img] = e;
+  if (pos == 0 && cb == 0) p.xe[img] = pair_word(e, mx, 0);
+#pragma unroll
+  for (int j = 0; j < 16; j++)
+    if (!in || c0 + j >= p.c) v[j >> 3][j & 7] = 0.f;
+  const unsigned below = pair_small_below(e);
+  unsigned mn = ~0u;
+#pragma unroll
+  for (int j = 0; j < 16; j++) mn = min(mn, pair_bits1(v[j >> 3][j & 7]));
+  if (__ballot(mn < below)) {  // uniform; few waves of ordinary data
+    int small = 0;
+#pragma unroll
+    for (int j = 0; j < 16; j++) small += pair_bits1(v[j >> 3][j & 7]) < below;
+    for (int o = 32; o > 0; o >>= 1) small += __shfl_xor(small, o);
+    if (lane == 0) atomicAdd(&p.xn[img * kCountStride], small);
+  }
   if (pos >= p.win_sp) return;
   uint4 *d = p.xi + ((int64_t)img * p.cb + cb) * p.win_sp * 4 + 2 * pos;
 #pragma unroll
   for (int h = 0; h < 2; h++) {
-#pragma unroll
-    for (int j = 0; j < 8; j++)
-      if (!in || c0 + 8 * h + j >= p.c) v[h][j] = 0.f;
     half8 hi, lo;
     pair_split8(v[h], e, &hi, &lo);
     d[h] = __builtin_bit_cast(uint4, hi);
@@ -119,24 +156,46 @@ __global__ __launch_bounds__(256) void k_conv_pair_x(const ConvPair p) {
   }
 }
 
-// The 32 x 32 block of channels m0 .. and columns of which lane l's is (img,
-// window origin oz, oy, ox), on fp32 MFMA straight from the tensors (marked
-// filters or images).
+// One wave's quarter of the sums of the 32 x 32 block of channels m0 .. and
+// columns of which lane l's is (img, window origin oz, oy, ox), on fp32 MFMA
+// straight from the tensors: steps of 16 channels at one tap, MFMA i of a step
+// channel 2 i for lanes 0-31 and 2 i + 1 for 32-63, the next step's loads in
+// flight.  Channels past m repeat the last one; nobody stores their sums.
 __device__ inline float16v conv_f32_tile(const ConvPair &p, int m0, int img, int oz, int oy, int ox,
-                                         int lane) {
-  const int m = m0 + (lane & 31), K = p.c * p.taps;
-  float16v acc = {};
-  for (int k0 = 0; k0 < K; k0 += 2) {
-    const int k = k0 + (lane >> 5);
-    const int c = k / p.taps, r = k - c * p.taps;
-    const int kx = r % p.ker[2], ky = r / p.ker[2] % p.ker[1], kz = r / p.ker[2] / p.ker[1];
+                                         int wave, int lane) {
+  const int h = lane >> 5, real = p.cb * p.taps, per = (real + 3) / 4;
+  const int s0 = wave * per, s1 = min(real, s0 + per);
+  const float *w = p.w + (int64_t)min(m0 + (lane & 31), p.m - 1) * p.c * p.taps;
+  const float *x = p.x + (int64_t)img * p.c * p.in_sp;
+  float a[2][8], b[2][8];
+  auto load = [&](int d, int s) __attribute__((always_inline)) {
+    const int c0 = s / p.taps * 16, tap = s % p.taps;
+    const int kx = tap % p.ker[2], ky = tap / p.ker[2] % p.ker[1], kz = tap / p.ker[2] / p.ker[1];
     const int iz = oz + kz * p.dil[0], iy = oy + ky * p.dil[1], ix = ox + kx * p.dil[2];
-    const bool ok = k < K && (unsigned)iz < (unsigned)p.in[0] && (unsigned)iy < (unsigned)p.in[1] &&
+    const bool ok = (unsigned)iz < (unsigned)p.in[0] && (unsigned)iy < (unsigned)p.in[1] &&
                     (unsigned)ix < (unsigned)p.in[2];
-    const float a = k < K && m < p.m ? p.w[(int64_t)m * K + k] : 0.f;
-    const float b =
-        ok ? p.x[((int64_t)img * p.c + c) * p.in_sp + (iz * p.in[1] + iy) * p.in[2] + ix] : 0.f;
-    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, acc, 0, 0, 0);
+    const float *xt = x + (ok ? (iz * p.in[1] + iy) * p.in[2] + ix : 0);
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+      const int ch = c0 + 2 * j + h, cc = min(ch, p.c - 1);
+      const float av = w[cc * p.taps + tap], bv = xt[(int64_t)cc * p.in_sp];
+      a[d][j] = ch < p.c ? av : 0.f;
+      b[d][j] = ch < p.c && ok ? bv : 0.f;
+    }
+  };
+  float16v acc = {};
+  auto step = [&](int d) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < 8; j++)
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[d][j], b[d][j], acc, 0, 0, 0);
+  };
+  if (s0 >= s1) return acc;
+  load(0, s0);
+  for (int s = s0; s < s1; s += 2) {
+    load(1, min(s + 1, s1 - 1));
+    step(0);
+    load(0, min(s + 2, s1 - 1));
+    if (s + 1 < s1) step(1);
   }
   return acc;
 }
@@ -150,6 +209,7 @@ __global__ __launch_bounds__(256, 2) void k_conv_pair(const ConvPair p) {
   __shared__ float4v part[4][4][4][64];
   __shared__ int exps[64];
   __shared__ float bias[64];
+  __shared__ int count;
   const int t = threadIdx.x, lane = t & 63, l32 = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   int tr, tc;
@@ -172,11 +232,13 @@ __global__ __launch_bounds__(256, 2) void k_conv_pair(const ConvPair p) {
   const int m0 = tr * 64, cols = p.n * p.out_sp, ns = p.ns, per = ns / 4;
   if (t < 64) {
     exps[t] = p.we[m0 + t];
+    const bool some = __ballot(pair_word_small(exps[t]) > 0) != 0;
+    if (t == 0) count = some;
     bias[t] = p.bias && m0 + t < p.m ? p.bias[m0 + t] : 0.f;
   }
   // The lane's column in each of the tile's two 32-column blocks: image,
   // output position and window origin.
-  int col[2], img[2], pos[2], oz[2], oy[2], ox[2], eb[2];
+  int col[2], img[2], pos[2], oz[2], oy[2], ox[2], eb[2], nb[2];
   unsigned vb[2];
 #pragma unroll
   for (int j = 0; j < 2; j++) {
@@ -188,6 +250,7 @@ __global__ __launch_bounds__(256, 2) void k_conv_pair(const ConvPair p) {
     oy[j] = pos[j] / p.out[2] % p.out[1] * p.str[1];
     oz[j] = pos[j] / p.out[2] / p.out[1] * p.str[0];
     eb[j] = p.xe[img[j]];
+    nb[j] = p.xn[img[j] * kCountStride];
     vb[j] = (unsigned)(img[j] * p.cb * p.win_sp * 64 +
                        ((oz[j] * p.win[1] + oy[j]) * p.win[2] + ox[j]) * 32 + 16 * h);
   }
@@ -229,43 +292,65 @@ __global__ __launch_bounds__(256, 2) void k_conv_pair(const ConvPair p) {
   };
   float16v s1[2][2];
   pair_sums(a, b, per, s1, load);
-  // (The barrier of the sum also publishes exps and bias.)
+  // (The barrier of the sum also publishes exps, bias and count.)
   const float16v sum = pair_reduce(part, wave, lane, s1);
   const int i = wave >> 1, j = wave & 1;
-  if (m0 + 32 * i >= p.m || tc * 64 + 32 * j >= cols) return;
+  const bool mine = m0 + 32 * i < p.m && tc * 64 + 32 * j < cols;
   const int cj = j ? col[1] : col[0], ij = j ? img[1] : img[0], pj = j ? pos[1] : pos[0];
-  const int ej = j ? eb[1] : eb[0];
-  bool marked = ej == kMarked;
-  int ea[16];
+  // A window has at most its own products' number of the image's small elements.
 #pragma unroll
-  for (int v = 0; v < 16; v++) {
-    ea[v] = exps[32 * i + 4 * h + 8 * (v >> 2) + (v & 3)];
-    marked |= ea[v] == kMarked;
-  }
-  float16v e = {};
-  if (__builtin_expect(__ballot(marked) != 0, 0))
-    e = conv_f32_tile(p, m0 + 32 * i, ij, (j ? oz[1] : oz[0]) - p.pad[0],
-                      (j ? oy[1] : oy[0]) - p.pad[1], (j ? ox[1] : ox[0]) - p.pad[2], lane);
+  for (int k = 0; k < 2; k++)
+    if (pair_word_small(eb[k]) == 0) eb[k] += min(nb[k], p.c * p.taps) * 1024;
+  const int wj = j ? eb[1] : eb[0];
+  int wa[16];
+#pragma unroll
+  for (int v = 0; v < 16; v++) wa[v] = exps[32 * i + 4 * h + 8 * (v >> 2) + (v & 3)];
+  // Without small elements in the tile's filters and images no output is redone.
+  const bool check =  // uniform: every wave holds the tile's columns
+      count != 0 || __ballot(pair_word_small(eb[0]) > 0 || pair_word_small(eb[1]) > 0) != 0;
+  const unsigned mask = check && mine ? pair_mask(part, wave, lane, wa, wj) : 0u;
   const __amdgpu_buffer_rsrc_t ry = rsrc(p.y);
+  // The outputs in `which`; stores of the others go past the resource and are
+  // dropped in hardware.
+  auto finish = [&](const float16v &s, unsigned which) __attribute__((always_inline)) {
 #pragma unroll
-  for (int v = 0; v < 16; v++) {
-    const int lr = 32 * i + 4 * h + 8 * (v >> 2) + (v & 3);
-    float y = ldexpf(sum[v], -(ea[v] + ej));
-    if (ea[v] == kMarked || ej == kMarked) y = e[v];
-    if (p.bias) y += bias[lr];
-    __builtin_amdgcn_raw_buffer_store_b32(
-        __builtin_bit_cast(unsigned, y), ry,
-        m0 + lr < p.m && cj < cols ? (unsigned)((ij * p.m + m0 + lr) * p.out_sp + pj) * 4u
-                                   : 0x80000000u,
-        0, 0);
+    for (int v = 0; v < 16; v++) {
+      const int lr = 32 * i + 4 * h + 8 * (v >> 2) + (v & 3);
+      const float y = p.bias ? s[v] + bias[lr] : s[v];
+      __builtin_amdgcn_raw_buffer_store_b32(
+          __builtin_bit_cast(unsigned, y), ry,
+          m0 + lr < p.m && cj < cols && (which >> v & 1)
+              ? (unsigned)((ij * p.m + m0 + lr) * p.out_sp + pj) * 4u
+              : 0x80000000u,
+          0, 0);
+    }
+  };
+  if (mine) {
+    float16v s;
+#pragma unroll
+    for (int v = 0; v < 16; v++)
+      s[v] = ldexpf(sum[v], -(pair_word_exp(wa[v]) + pair_word_exp(wj)));
+    finish(s, ~mask);
   }
+  if (!check) return;
+  // (Copies: arrays indexed by a lambda's argument would be kept in LDS.)
+  const int i0 = img[0], i1 = img[1], z0 = oz[0], z1 = oz[1], y0 = oy[0], y1 = oy[1], x0 = ox[0],
+            x1 = ox[1];
+  pair_redo(
+      part, wave, lane, mask,
+      [=](int q, int w) __attribute__((always_inline)) {
+        const bool k = q & 1;
+        return conv_f32_tile(p, m0 + 32 * (q >> 1), k ? i1 : i0, (k ? z1 : z0) - p.pad[0],
+                             (k ? y1 : y0) - p.pad[1], (k ? x1 : x0) - p.pad[2], w, lane);
+      },
+      [&](const float16v &s) __attribute__((always_inline)) { finish(s, mask); });
 }
 
 struct Plan {
   bool ok = false;
   ConvPair q{};
   int64_t nb = 0;  // images per round of launches
-  size_t off_we = 0, off_xi = 0, off_xe = 0, off_part = 0, total = 0;
+  size_t off_we = 0, off_xi = 0, off_xe = 0, off_xn = 0, off_part = 0, total = 0;
 };
 
 Plan plan(const mg_conv_problem &p) {
@@ -301,7 +386,7 @@ Plan plan(const mg_conv_problem &p) {
       (p.m * taps < 128 && p.n * p.c * in * 4 > (int64_t)8 << 20))
     return r;
   // 32-bit offsets throughout, and the filter rows as laid out.
-  if (p.w_ms != p.c * taps || p.w_cs != taps || p.c * taps >= lim || p.c * in >= lim ||
+  if (p.w_ms != p.c * taps || p.w_cs != taps || p.c * taps > kPairMaxSmall || p.c * in >= lim ||
       mp * ns * 64 >= 4 * lim || ns * 2048 * 2 >= 4 * lim || img >= 4 * lim || p.m * out >= lim ||
       (win + 255) / 256 > 0x7fffff || cb > 65535)
     return r;
@@ -321,6 +406,8 @@ Plan plan(const mg_conv_problem &p) {
   off += mg_align((size_t)(r.nb * img));
   r.off_xe = off;
   off += mg_align((size_t)r.nb * 4);
+  r.off_xn = off;
+  off += (size_t)r.nb * kCountStride * 4;
   r.off_part = off;
   off += mg_align((size_t)(r.nb * q.chunks) * 4);
   r.total = off;
@@ -345,6 +432,7 @@ mg_status mg_conv_pair_run(mg_ctx *ctx, const mg_conv_problem &p, void *ws) {
   q.we = reinterpret_cast<int *>(base + r.off_we);
   q.xi = reinterpret_cast<uint4 *>(base + r.off_xi);
   q.xe = reinterpret_cast<int *>(base + r.off_xe);
+  q.xn = reinterpret_cast<int *>(base + r.off_xn);
   q.part = reinterpret_cast<unsigned *>(base + r.off_part);
   const int mp = (q.m + 63) / 64 * 64;
   for (int64_t n0 = 0; n0 < p.n; n0 += r.nb) {

@@ -2,17 +2,19 @@
 //
 // Every operand row (a row of A, a column of B) is scaled by a power of two
 // that puts its largest magnitude in [2^14, 2^15) and each element x is
-// carried as hi = fp16(x) and lo = fp16((x - hi) 2^11).  hi and lo hold 23
-// significant bits of x (fp32's 24 less half a bit on average) for every
-// element down to 2^-29 of the row's largest, and the smaller ones to 2^-51
-// of it.  The product is hi hi' + 2^-11 (hi lo' + lo hi'), each sum in an
-// fp32 accumulator of its own; lo lo' (2^-24 of the product at most) is left
+// carried as hi = fp16(x) and lo = fp16((x - hi) 2^11).  hi and lo are within
+// 2^-23 of x (fp32's 24 bits less half a bit on average) for every element down
+// to 2^-28 of the row's largest; rows with smaller ones count them.
+// The product is hi hi' + 2^-11 (hi lo' + lo hi'), each sum in an
+// fp32 accumulator of its own; lo lo' (2^-22 of the product at most) is left
 // out.  Three v_mfma_f32_32x32x16_f16 take the place of eight
 // v_mfma_f32_32x32x2_f32 on 1/5 of their matrix-core time, and the leading
 // sum is rounded once per 16 k instead of once per 2.
 //
-// Rows that hold Inf or NaN are marked; their outputs are computed on fp32
-// MFMA from the fp32 operands (f32_tile).
+// Outputs that this cannot give to fp32's accuracy are computed on fp32 MFMA
+// from the fp32 operands (f32_tile): those of rows that hold Inf or NaN, and sums
+// of products so small that the lost parts of small elements could show in them
+// (pair_mask).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -24,7 +26,7 @@ namespace {
 // Pair images of X [R, K] (row-major, K contiguous): per 32 rows and 16 k a
 // hi and a lo fragment of 1 KiB in MFMA operand order, [r32][k16][hi|lo][32 h
 // + r][8] for row r and k = 16 k16 + 8 h .. +7; zeros past R and K.  ex[row]
-// is the row's exponent (kMarked: Inf or NaN, digits zero).
+// is the row's exponent and count of small elements (pair_word).
 // TPR threads per row, 256 / TPR rows per workgroup; UL > 0: a thread keeps
 // its UL octets in registers between the row maximum and the split (K <= 8
 // TPR UL), UL = 0 reads the row twice.  Bound by memory at large R (4096 x 1536:
@@ -50,11 +52,15 @@ __global__ __launch_bounds__(256) void k_pair_split(const float *__restrict__ X,
       for (int i = 0; i < 8; i++) v[i] = row < R && k0 + i < K ? x[k0 + i] : 0.f;
     }
   };
-  // Largest magnitude as bits: ordered as integers, Inf and NaN largest.
-  unsigned mx = 0;
+  // Largest and smallest nonzero magnitude as bits: ordered as integers, Inf
+  // and NaN largest.
+  unsigned mx = 0, mn = ~0u;
   auto amax = [&](const float v[8]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < 8; i++) mx = max(mx, __builtin_bit_cast(unsigned, v[i]) & 0x7fffffffu);
+    for (int i = 0; i < 8; i++) {
+      mx = max(mx, __builtin_bit_cast(unsigned, v[i]) & 0x7fffffffu);
+      mn = min(mn, pair_bits1(v[i]));
+    }
   };
   const int no = 2 * nk;
   float v[UL ? UL : 1][8];
@@ -77,9 +83,14 @@ __global__ __launch_bounds__(256) void k_pair_split(const float *__restrict__ X,
     mx = max(max(wmx[0], wmx[1]), max(wmx[2], wmx[3]));
   }
   const int e = pair_exponent(mx);
-  if (u == 0) ex[row] = e;
+  // (The thread's own smallest spares the count where there is none.)
+  const unsigned below = pair_small_below(e);
+  int small = 0;
   auto store = [&](int o, const float w[8]) __attribute__((always_inline)) {
     if (o >= no) return;
+    if (mn < below)
+#pragma unroll
+      for (int i = 0; i < 8; i++) small += pair_bits1(w[i]) < below;
     half8 hi, lo;
     pair_split8(w, e, &hi, &lo);
     uint4 *d = img + (((row >> 5) * nk + (o >> 1)) * 2) * 64 + 32 * (o & 1) + (row & 31);
@@ -95,35 +106,71 @@ __global__ __launch_bounds__(256) void k_pair_split(const float *__restrict__ X,
       store(o, v[0]);
     }
   }
+  for (int o = std::min(TPR, 64) / 2; o > 0; o >>= 1) small += __shfl_xor(small, o);
+  if constexpr (TPR > 64) {
+    __shared__ int wsm[4];
+    if ((t & 63) == 0) wsm[t >> 6] = small;
+    __syncthreads();
+    small = wsm[0] + wsm[1] + wsm[2] + wsm[3];
+  }
+  if (u == 0) ex[row] = pair_word(e, mx, small);
 }
 
-// One 32 x 32 output tile of A [M, K] . B [N, K]^T on fp32 MFMA (k pairs in
-// order), operands read from memory with bounds checks.
+// One wave's quarter of the sums of a 32 x 32 output tile of A [M, K] . B [N,
+// K]^T on fp32 MFMA, operands read straight from memory: MFMA i of eight k holds
+// k = i (lanes 0-31) and 4 + i (lanes 32-63), so that a lane's four k are one
+// 16-byte load (vec: rows are aligned for it).  The next 32 k are on their way
+// during the products.  Rows past M and columns past N repeat the last one;
+// nobody stores their sums.
 __device__ inline float16v f32_tile(const float *__restrict__ A, const float *__restrict__ B,
-                                    int64_t M, int64_t N, int64_t K, int64_t r0, int64_t c0,
-                                    int lane) {
-  const int64_t r = r0 + (lane & 31), c = c0 + (lane & 31);
-  float16v acc = {};
-  for (int64_t kb = 0; kb < K; kb += 16) {
-    float a[8], b[8];
+                                    int64_t M, int64_t N, int64_t K, int vec, int64_t r0,
+                                    int64_t c0, int wave, int lane) {
+  const float *pa = A + min(r0 + (lane & 31), M - 1) * K, *pb = B + min(c0 + (lane & 31), N - 1) * K;
+  const int64_t per = (K + 127) / 128 * 32, kend = min(K, (wave + 1) * per);
+  const int64_t k0 = 4 * (lane >> 5);
+  float4v a[2][4], b[2][4];
+  auto load = [&](int d, int64_t kb) __attribute__((always_inline)) {
+    if (vec && kb + 32 <= kend) {
 #pragma unroll
-    for (int s = 0; s < 8; s++) {
-      const int64_t k = kb + 2 * s + (lane >> 5);
-      a[s] = r < M && k < K ? A[r * K + k] : 0.f;
-      b[s] = c < N && k < K ? B[c * K + k] : 0.f;
+      for (int j = 0; j < 4; j++) {
+        a[d][j] = *reinterpret_cast<const float4v *>(pa + kb + 8 * j + k0);
+        b[d][j] = *reinterpret_cast<const float4v *>(pb + kb + 8 * j + k0);
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const int64_t k = kb + 8 * j + k0 + i;
+          a[d][j][i] = k < kend ? pa[k] : 0.f;
+          b[d][j][i] = k < kend ? pb[k] : 0.f;
+        }
     }
+  };
+  float16v acc = {};
+  auto step = [&](int d) __attribute__((always_inline)) {
 #pragma unroll
-    for (int s = 0; s < 8; s++)
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s], b[s], acc, 0, 0, 0);
+    for (int j = 0; j < 4; j++)
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[d][j][i], b[d][j][i], acc, 0, 0, 0);
+  };
+  load(0, wave * per);
+  for (int64_t kb = wave * per; kb < kend; kb += 64) {
+    load(1, kb + 32);
+    step(0);
+    load(0, kb + 64);
+    step(1);
   }
   return acc;
 }
 
 struct PairArgs {
   const uint4 *ai, *bi;     // pair images
-  const int *ae, *be;       // row exponents
-  const float *a, *b;       // the fp32 operands (marked rows)
+  const int *ae, *be;       // row exponents and counts (pair_word)
+  const float *a, *b;       // the fp32 operands (f32_tile)
   int64_t M, N, K;
+  int vec;                  // their rows are 16-byte aligned
   int nk, nx, pr, pc;       // 16-k steps; tile grid and its XCD cut
   float alpha, beta;
   const float *c;
@@ -148,6 +195,7 @@ __global__ __launch_bounds__(256, 2) void k_pair_gemm(const PairArgs p) {
   constexpr int T = 64, KW = 4;
   __shared__ float4v part[KW][4][4][64];  // [wave][32 x 32 block][v / 4][lane]
   __shared__ __attribute__((aligned(16))) int exps[2 * T];
+  __shared__ int counts[2];
   const int t = threadIdx.x, lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   int tr, tc;
@@ -190,36 +238,43 @@ __global__ __launch_bounds__(256, 2) void k_pair_gemm(const PairArgs p) {
                                                          (i * nk + k) * 2048, 0));
       }
   };
-  // The tile's exponents (images reach to whole 64-row blocks) and a column's
+  // The tile's words (images reach to whole 64-row blocks) and a column's
   // C where C is a row: read here, not in the epilogue, where each would be a
   // round trip of its own.
   const int l32 = lane & 31, h = lane >> 5;
-  if (t < 2 * T) exps[t] = t < T ? p.ae[r0 + t] : p.be[c0 + t - T];
+  if (t < 2 * T) {  // waves 0 and 1
+    exps[t] = t < T ? p.ae[r0 + t] : p.be[c0 + t - T];
+    const bool some = __ballot(pair_word_small(exps[t]) > 0) != 0;
+    if (lane == 0) counts[wave] = some;
+  }
   float cb[2] = {0.f, 0.f};
   if (p.c && p.c_rs == 0)
 #pragma unroll
     for (int j = 0; j < 2; j++) cb[j] = p.c[min(c0 + 32 * j + l32, p.N - 1) * p.c_cs];
   float16v s1[2][2];
   pair_sums(a, b, per, s1, load);
-  // y = sum 2^-(ea + eb) of the 32 x 32 block (i, j) of the tile: lane
-  // l holds column l % 32 and rows 8 (v / 4) + 4 (l / 32) + v % 4.  Stores
-  // past M or N go past the resource and are dropped in hardware.
-  auto finish = [&](const float16v &sum, int i, int j) __attribute__((always_inline)) {
-    const int64_t tr0 = r0 + 32 * i, tc0 = c0 + 32 * j;
-    if (tr0 >= p.M || tc0 >= p.N) return;
-    const int64_t col = tc0 + l32, rw = tr0 + 4 * h;
-    const int eb = exps[T + 32 * j + l32];
-    int ea[16];
-    bool marked = eb == kMarked;
+  // (The barrier of the sum also publishes exps and counts.)
+  const float16v sum = pair_reduce(part, wave, lane, s1);
+  // This wave's 32 x 32 block (i, j) of the tile: lane l holds column l % 32
+  // and rows 8 (v / 4) + 4 (l / 32) + v % 4.
+  const int i = wave >> 1, j = wave & 1;
+  const int64_t tr0 = r0 + 32 * i, tc0 = c0 + 32 * j;
+  const bool mine = tr0 < p.M && tc0 < p.N;
+  const int wb = exps[T + 32 * j + l32];
+  int wa[16];
 #pragma unroll
-    for (int v = 0; v < 16; v += 4) {
-      const int4 x = *reinterpret_cast<const int4 *>(&exps[32 * i + 4 * h + 2 * v]);
-      ea[v] = x.x, ea[v + 1] = x.y, ea[v + 2] = x.z, ea[v + 3] = x.w;
-      marked |= x.x == kMarked || x.y == kMarked || x.z == kMarked || x.w == kMarked;
-    }
-    float16v e = {};
-    if (__builtin_expect(__ballot(marked) != 0, 0))
-      e = f32_tile(p.a, p.b, p.M, p.N, p.K, tr0, tc0, lane);
+  for (int v = 0; v < 16; v += 4) {
+    const int4 x = *reinterpret_cast<const int4 *>(&exps[32 * i + 4 * h + 2 * v]);
+    wa[v] = x.x, wa[v + 1] = x.y, wa[v + 2] = x.z, wa[v + 3] = x.w;
+  }
+  // Without small elements in the tile's rows and columns no output is redone (a
+  // barrier at the end of every workgroup took 3 us of FFN1's 32).
+  const bool check = (counts[0] | counts[1]) != 0;  // uniform
+  const unsigned mask = check && mine ? pair_mask(part, wave, lane, wa, wb) : 0u;
+  // y = alpha sum + beta C of the outputs in `which`.  Stores of the others, and
+  // past M or N, go past the resource and are dropped in hardware.
+  auto finish = [&](const float16v &s, unsigned which) __attribute__((always_inline)) {
+    const int64_t col = tc0 + l32, rw = tr0 + 4 * h;
     float cv[16];
 #pragma unroll
     for (int v = 0; v < 16; v++) cv[v] = cb[j];
@@ -234,17 +289,30 @@ __global__ __launch_bounds__(256, 2) void k_pair_gemm(const PairArgs p) {
 #pragma unroll
     for (int v = 0; v < 16; v++) {
       const int lr = 4 * h + 8 * (v >> 2) + (v & 3);
-      float y = ldexpf(sum[v], -(ea[v] + eb));
-      if (ea[v] == kMarked || eb == kMarked) y = e[v];
+      float y = s[v];
       if (p.alpha != 1.f) y = p.alpha * y;
       if (p.c) y = y + (p.beta != 1.f ? p.beta * cv[v] : cv[v]);
-      __builtin_amdgcn_raw_buffer_store_b32(
-          __builtin_bit_cast(unsigned, y), ry,
-          tr0 + lr < p.M && col < p.N ? (unsigned)(lr * (int)p.ldy + l32) * 4u : 0x80000000u, 0, 0);
+      const bool st = tr0 + lr < p.M && col < p.N && (which >> v & 1);
+      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, y), ry,
+                                            st ? (unsigned)(lr * (int)p.ldy + l32) * 4u : 0x80000000u,
+                                            0, 0);
     }
   };
-  // (The barrier of the sum also publishes exps.)
-  finish(pair_reduce(part, wave, lane, s1), wave >> 1, wave & 1);
+  if (mine) {
+    float16v s;
+#pragma unroll
+    for (int v = 0; v < 16; v++)
+      s[v] = ldexpf(sum[v], -(pair_word_exp(wa[v]) + pair_word_exp(wb)));
+    finish(s, ~mask);
+  }
+  if (!check) return;
+  pair_redo(
+      part, wave, lane, mask,
+      [&](int q, int w) __attribute__((always_inline)) {
+        return f32_tile(p.a, p.b, p.M, p.N, p.K, p.vec, r0 + 32 * (q >> 1), c0 + 32 * (q & 1), w,
+                        lane);
+      },
+      [&](const float16v &s) __attribute__((always_inline)) { finish(s, mask); });
 }
 
 }  // namespace
@@ -302,6 +370,8 @@ mg_status mg_pair_run(mg_ctx *ctx, const mg_f32_problem &p, const float *a_dev,
   q.be = reinterpret_cast<const int *>(static_cast<const char *>(b_img) + mg_align((size_t)(np * q.nk * 64)));
   q.a = a_dev;
   q.b = b_dev;
+  q.vec = p.K % 4 == 0 && reinterpret_cast<uintptr_t>(a_dev) % 16 == 0 &&
+          reinterpret_cast<uintptr_t>(b_dev) % 16 == 0;
   q.M = p.M;
   q.N = p.N;
   q.K = p.K;

@@ -1,6 +1,7 @@
 """fp32 Conv on fp16 digit pairs against float64, at the edges of its 16-channel
-blocks, 64 x 64 tiles and padded windows, over 1-D to 3-D geometries, with Inf
-and NaN, and without its workspace (the fp32 MFMA kernel)."""
+blocks, 64 x 64 tiles and padded windows, over 1-D to 3-D geometries, over wide
+ranges within an image or a filter, with Inf and NaN, and without its workspace
+(the fp32 MFMA kernel)."""
 import numpy as np
 import pytest
 
@@ -33,15 +34,17 @@ def reference(x, w, b, stride, pads, dil):
             conv64(np.abs(x), np.abs(w), stride, pads, dil) + np.abs(b))
 
 
-def check(y, x, w, b, stride, pads, dil):
-    """Two digits leave 2^-23 of an operand, lo lo' 2^-24 of a product, and
-    each of the K / 16 additions (and the last few) 2^-23 of the sum."""
+def check(y, x, w, b, stride, pads, dil, redone=False):
+    """Two digits leave 2^-23 of an operand, lo lo' 2^-22 of a product, what
+    small elements lose 2^-21 of the sum, and each of the K / 16 additions (and
+    the last few) 2^-23 of the sum.  Outputs computed on fp32 MFMA add K / 2
+    times, each 2^-24."""
     want, size = reference(x, w, b, stride, pads, dil)
     k = np.prod(w.shape[1:])
     steps = -(-w.shape[1] // 16) * np.prod(w.shape[2:])
     assert k >= 256
     assert y.shape == want.shape
-    assert (np.abs(y - want) <= (steps + 12) * 2.0**-23 * size).all()
+    assert (np.abs(y - want) <= (steps + 12 + k / 4 * redone) * 2.0**-23 * size).all()
 
 
 CASES = [  # x, w, stride, pads, dilation
@@ -98,6 +101,35 @@ def test_inf_and_nan(ops):
     rest = np.setdiff1d(np.arange(130), [65])
     np.testing.assert_array_equal(y[:, rest], clean[:, rest])
     np.testing.assert_array_equal(y[:, 65], np.sign(x[:, 0]) * np.float32(np.inf))
+
+
+@pytest.mark.parametrize("big", [1e6, 1e12, 1e20, -3.4028235e38])
+@pytest.mark.parametrize("case", CASES[1:4] + CASES[7:], ids=lambda c: "x".join(map(str, c[0] + c[1])))
+def test_large_value_in_a_corner(ops, case, big):
+    # One value of an image (and one of a filter) far above the others: the
+    # windows (channels) that do not hold it are as good as without it.
+    x, w, b = (t / 10 for t in draw(case, 3))
+    whole = x.copy()
+    x[0, 0].flat[0] = big
+    x[-1, -1].flat[-1] = big
+    v = w.copy()
+    v[len(v) // 2, 0].flat[0] = big
+    args = dict(strides=list(case[2]), pads=list(case[3]), dilations=list(case[4]))
+    check(ops.op_conv(x, w, b, **args), x, w, b, *case[2:], redone=True)
+    check(ops.op_conv(whole, v, b, **args), whole, v, b, *case[2:], redone=True)
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "x".join(map(str, c[0] + c[1])))
+def test_opposite_ranges(ops, case):
+    # Channels over 2^80 in the input and the other way round in the filters; an
+    # image and a filter of zeros.
+    x, w, b = draw(case, 4)
+    s = np.random.default_rng(5).integers(-40, 41, x.shape[1]).reshape((1, -1) + (1,) * (x.ndim - 2))
+    x, w = (x * 2.0**s).astype(np.float32), (w * 2.0**-s).astype(np.float32)
+    x[-1] *= len(x) == 1
+    w[-1] *= len(w) == 1
+    y = ops.op_conv(x, w, b, strides=list(case[2]), pads=list(case[3]), dilations=list(case[4]))
+    check(y, x, w, b, *case[2:], redone=True)
 
 
 def test_without_workspace(ops):

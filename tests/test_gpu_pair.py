@@ -1,7 +1,8 @@
 """Weight Gemms on fp16 digit pairs (F32Weight.gemm) against float64, at the
 edges of their 64 x 64 tiles and 64-k padding, over every plan of the digit
-split, over wide exponent ranges, with Inf and NaN operands (the fp32 form of
-the tile) and without the workspace they would like to have (the fp32 MFMA
+split, over wide exponent ranges within a row (outputs that lost parts of small
+elements could show in) and with Inf and NaN operands, both on the fp32 form of
+the tile, and without the workspace they would like to have (the fp32 MFMA
 kernel)."""
 import numpy as np
 import pytest
@@ -16,10 +17,10 @@ def ops():
 
 
 def check(y, a, w, c=0.0, alpha=1.0, beta=1.0):
-    """Element by element: the two digits leave 2^-23 of an operand, lo lo'
-    2^-24 of a product, and each of the K / 16 additions per output (and the
-    few that join the shares, scale and add C) at most 2^-23 of what has been
-    added, all of it at most sum |a| |w|."""
+    """Element by element: the digits leave 2^-23 of an operand, lo lo' 2^-22
+    of a product, what small elements lose 2^-21 of the sum, and each of the
+    K / 16 additions per output (and the few that join the shares, scale and add
+    C) at most 2^-23 of what has been added, all of it at most sum |a| |w|."""
     a, w = a.astype(np.float64), w.astype(np.float64)
     want = alpha * (a @ w.T) + beta * c
     size = abs(alpha) * (np.abs(a) @ np.abs(w).T) + np.abs(beta * c)
@@ -126,3 +127,85 @@ def test_image_bytes(ops):
         fw = ops.F32Weight(np.zeros((n, k), np.float32), trans_b=True)
         assert 4 * n * k <= fw.info()[2] <= 12 * n * k + (1 << 20)
         fw.release()
+
+
+# Two elements of a row, two of a column: the large one meets a zero or a small
+# factor, so that the small one is the result.
+LOST = [((1e20, 1), (0, 1)), ((3.4028235e38, 1.5), (0, 1)), ((1e8, 1e-8), (1e-8, 1e8)),
+        ((1e12, 1.2345678), (0, 1)), ((1e6, 1.2345678e-6), (0, 1)), ((1e-30, 1e-45), (0, 1e30)),
+        ((0, 1), (1e20, 1))]
+
+
+@pytest.mark.parametrize("k", [256, 259, 513])
+def test_large_beside_small(ops, k):
+    rng = np.random.default_rng(k)
+    n = len(LOST)
+    a, w = np.zeros((66, k), np.float32), np.zeros((n, k), np.float32)
+    for i, (x, y) in enumerate(LOST):
+        at = rng.choice(k, 2, replace=False)
+        a[i, at], a[-1 - i, at] = x, x
+        w[i, at] = y
+    fw = ops.F32Weight(w, trans_b=True)
+    y = fw.gemm(a)
+    fw.release()
+    check(y, a, w)
+    for i, (x, z) in enumerate(LOST):
+        want = np.dot(np.float32(x).astype(np.float64), np.float32(z).astype(np.float64))
+        assert y[i, i] == y[-1 - i, i] == np.float32(want), (i, y[i, i], want)
+
+
+@pytest.mark.parametrize("k,off", [(256, 0), (320, 1), (301, 0)])
+def test_ranges_within_a_row(ops, k, off):
+    # Elements of a row over 2^80 against single elements (a permutation) and
+    # against columns of the opposite range, whose products are all alike; a
+    # zero row and a row whose one large element meets a zero.
+    rng = np.random.default_rng(8)
+    m = 70
+    s = rng.integers(-40, 41, k)
+    a = (rng.standard_normal((m, k)) * 2.0**s).astype(np.float32)
+    a[3], a[40, 5] = 0, 3e38
+    one = np.eye(k, dtype=np.float32)[rng.permutation(k)]
+    w = (rng.standard_normal((130, k)) * 2.0**-s).astype(np.float32)
+    w[:, 5] = 0
+    ad = ops.DeviceBuffer.from_array(np.concatenate([np.zeros(off, np.float32), a.ravel()]))
+    for b in (one, w):
+        fw = ops.F32Weight(b, trans_b=True)
+        yd = ops.DeviceBuffer(m * len(b) * 4)
+        fw.gemm_dev(ad.ptr + 4 * off, m, yd.ptr)
+        y = yd.to_array((m, len(b)), np.float32)
+        check(y, a, b)
+        assert (y[3] == 0).all()
+        if b is one:
+            want = a.astype(np.float64) @ one.T
+            assert (np.abs(y - want) <= 2.0**-22 * np.abs(want)).all()
+        fw.release()
+        yd.free()
+    ad.free()
+
+
+def test_inf_and_nan_beside_small(ops):
+    # As test_inf_and_nan, at a K of the pairs, with rows of zeros and of small
+    # elements among them: 0 Inf is NaN, as the sum in fp32 gives it.
+    rng = np.random.default_rng(9)
+    a = rng.standard_normal((100, 300)).astype(np.float32)
+    w = rng.standard_normal((90, 300)).astype(np.float32)
+    a[50] = 0
+    a[51, 7] = 1e30
+    w[20] = 0
+    v = w.copy()
+    v[11, 2], v[64, 64] = np.inf, np.nan
+    b = a.copy()
+    b[3, 7], b[40, 100] = -np.inf, np.nan
+    fw, fv = ops.F32Weight(w, trans_b=True), ops.F32Weight(v, trans_b=True)
+    clean, y, z = fw.gemm(a), fw.gemm(b), fv.gemm(a)
+    fw.release()
+    fv.release()
+    check(clean, a, w)
+    rows, cols = np.setdiff1d(np.arange(100), [3, 40]), np.setdiff1d(np.arange(90), [11, 64])
+    np.testing.assert_array_equal(y[rows], clean[rows])
+    with np.errstate(invalid="ignore"):
+        np.testing.assert_array_equal(y[3], w[:, 7] * np.float32(-np.inf))
+        assert np.isnan(y[40]).all()
+        np.testing.assert_array_equal(z[:, cols], clean[:, cols])
+        np.testing.assert_array_equal(z[:, 11], a[:, 2] * np.float32(np.inf))
+    assert np.isnan(z[:, 64]).all()
