@@ -356,7 +356,8 @@ struct Plan {
 Plan plan(const mg_conv_problem &p) {
   Plan r;
   if (p.xk != MG_CONV_F32 || p.trans || p.phased || p.group != 1) return r;
-  const int64_t lim = (int64_t)1 << 29;
+  // Elements of a round's output: its resource ends 16 bytes below 2^31.
+  const int64_t lim = (int64_t)1 << 29, out_max = lim - 4;
   int64_t win = 1, out = 1, in = 1, taps = 1;
   ConvPair &q = r.q;
   for (int d = 0; d < 3; d++) {
@@ -387,10 +388,10 @@ Plan plan(const mg_conv_problem &p) {
     return r;
   // 32-bit offsets throughout, and the filter rows as laid out.
   if (p.w_ms != p.c * taps || p.w_cs != taps || p.c * taps > kPairMaxSmall || p.c * in >= lim ||
-      mp * ns * 64 >= 4 * lim || ns * 2048 * 2 >= 4 * lim || img >= 4 * lim || p.m * out >= lim ||
+      mp * ns * 64 >= 4 * lim || ns * 2048 * 2 >= 4 * lim || img >= 4 * lim || p.m * out > out_max ||
       (win + 255) / 256 > 0x7fffff || cb > 65535)
     return r;
-  const int64_t fit = std::min<int64_t>((64ll << 20) / img, lim / (p.m * out));
+  const int64_t fit = std::min<int64_t>((64ll << 20) / img, out_max / (p.m * out));
   r.nb = std::max<int64_t>(1, std::min<int64_t>(p.n, std::min<int64_t>(fit, 65535)));
   q.c = (int)p.c, q.m = (int)p.m, q.taps = (int)taps, q.cb = (int)cb, q.ns = (int)ns;
   q.in_sp = (int)in, q.out_sp = (int)out, q.win_sp = (int)win;

@@ -132,6 +132,35 @@ def test_opposite_ranges(ops, case):
     check(y, x, w, b, *case[2:], redone=True)
 
 
+def test_two_gib_of_output(ops):
+    # Images that would fill a round's output to exactly 2^31 bytes.
+    n, c, size, m = 64, 32, 64, 2048
+    rng = np.random.default_rng(6)
+    x = rng.standard_normal((n, c, size, size)).astype(np.float32)
+    w = rng.standard_normal((m, c, 3, 3)).astype(np.float32)
+    xd, wd = ops.DeviceBuffer.from_array(x), ops.DeviceBuffer.from_array(w)
+    y = ops.DeviceBuffer(n * m * size * size * 4)
+    assert y.nbytes == 1 << 31
+
+    class Tail(ops.DeviceBuffer):
+        def __init__(self, image, channel):
+            self.ctx, self.ptr = y.ctx, y.ptr + (image * m + channel) * size * size * 4
+
+        def free(self):
+            pass
+
+    nan = np.full((size, size), np.nan, np.float32)
+    at = [(0, 0), (31, 1000), (62, m - 1), (63, 0), (63, m - 1)]
+    for i, o in at:
+        ops.check(ops.lib.mg_buffer_upload(y.ctx.handle, Tail(i, o).ptr, nan.ctypes.data, nan.nbytes))
+    ops.conv_f32_dev(xd.ptr, x.shape, wd.ptr, w.shape, y.ptr, strides=[1, 1], pads=[1] * 4)
+    for i, o in at:
+        got = Tail(i, o).to_array((1, 1, size, size), np.float32)
+        check(got, x[i:i + 1], w[o:o + 1], np.zeros(1, np.float32), (1, 1), (1, 1, 1, 1), (1, 1))
+    for d in (xd, wd, y):
+        d.free()
+
+
 def test_without_workspace(ops):
     case = CASES[2]
     x, w, b = draw(case, 2)
