@@ -389,14 +389,15 @@ mg_status mg_gemm_f32(mg_ctx *ctx, const float *a, const int64_t *a_shape,
  * lib/src/onnx_graph.dart:2159-2161 done once on upload).  Beside the fp32
  * values the weight keeps their fp16 digit pairs (4 more bytes per element with
  * N padded to 64 columns and K to 64, counted by mg_weight_info).  They are left
- * out for K > 2^18 - 64 or N >= 2^22, where the padding makes them more than
+ * out for K < 192, K > 2^18 - 64 or N >= 2^22, where the padding makes them more than
  * twice the weight plus a MiB, and where the device has no room. */
 mg_status mg_weight_f32_create(mg_ctx *ctx, const float *b, int64_t rows,
                                int64_t cols, int32_t trans_b, mg_weight **out);
 /* y[rows, N] = alpha * a[rows, K] . W + beta * C, C as in mg_gemm_f32 (may be
  * NULL).  With alpha = 1, beta = 0, C = NULL this is MatMul against an
  * initializer, including the shared-weight batch collapse
- * (lib/src/onnx_ops.dart:1728-1735).  Where the weight has digit pairs, the
+ * (lib/src/onnx_ops.dart:1728-1735).  Where the weight has digit pairs and
+ * they are faster (sums of 192 products and more, by a rule on rows, K and N), the
  * products are formed from them: every output is within 2^-21 of its sum of
  * |a| |b|, beside the rounding of the fp32 sums (closer than fp32 products on
  * ordinary data, whose sums round more often; outputs that need more, and those

@@ -1384,12 +1384,13 @@ mg_status gemm_w(mg_ctx *ctx, const float *a, bool a_dev_ptr, int64_t rows, int6
   const size_t oa = a_dev_ptr ? 0 : s.take((size_t)(rows * K) * 4);
   const size_t oc = (c && !c_dev_ptr) ? s.take((size_t)nc * 4) : 0;
   const size_t oy = y_dev_ptr ? 0 : s.take((size_t)(rows * w->N) * 4);
-  // On pair images where the weight has them and the images of A (row chunks
-  // of at most 64 MiB) can be had; else on the fp32 MFMA kernel, which needs
+  // On pair images where the weight has them, they pay, and the images of A (row
+  // chunks of at most 64 MiB) can be had; else on the fp32 MFMA kernel, which needs
   // less workspace or none.
   const int64_t chunk = MG_PAIR_CHUNK_BYTES / (int64_t)mg_pair_bytes(64, K) * 64;
   const size_t pb = mg_align(mg_pair_bytes(std::min(rows, chunk), K));
-  const bool pair = w->f32.pair && mg_ws_optional(ctx, s.off + pb);
+  const bool pair =
+      w->f32.pair && mg_pair_pays(rows, w->N, K) && mg_ws_optional(ctx, s.off + pb);
   q.kspl = pair ? 1 : mg_f32_ksplit(rows, K, 1);
   // Partials of at most 64 MiB: wider weights run in column chunks.
   if (q.kspl > 1)

@@ -341,8 +341,9 @@ bool mg_f32_xcd_cut(int64_t ny, int64_t nx, int *pr, int *pc, int64_t *per);
 // pair.hip) of an fp32 matrix of R rows of K contiguous elements, and y =
 // alpha A . B^T + beta C of one batch on the images of A [M, K] and B [N, K].
 size_t mg_pair_bytes(int64_t R, int64_t K);
-// Whether a weight [N, K] keeps pair images.
+// Whether a weight [N, K] keeps pair images, and whether M rows take them.
 bool mg_pair_keeps(int64_t N, int64_t K);
+bool mg_pair_pays(int64_t M, int64_t N, int64_t K);
 constexpr int64_t MG_PAIR_CHUNK_BYTES = 64 << 20;  // of A's images per round of launches
 mg_status mg_pair_split(mg_ctx *ctx, const float *x_dev, int64_t R, int64_t K, void *img);
 mg_status mg_pair_run(mg_ctx *ctx, const mg_f32_problem &p, const float *a_dev,

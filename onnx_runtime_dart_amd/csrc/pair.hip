@@ -31,7 +31,8 @@ namespace {
 // its UL octets in registers between the row maximum and the split (K <= 8
 // TPR UL), UL = 0 reads the row twice.  Bound by memory at large R (4096 x 1536:
 // 25 MB in, 25 MB out, 10.4 us, 4.8 TB/s) and by its launch and one round trip at small ones, so
-// rows of few workgroups take a whole workgroup each.
+// rows of few workgroups take a whole workgroup each (long rows in eights, whose
+// pieces fill whole lines: a call of 4096 x 4096 -> 1024 0.7 of the time).
 template <int TPR, int UL>
 __global__ __launch_bounds__(256) void k_pair_split(const float *__restrict__ X, int64_t R,
                                                     int64_t K, int nk, int vec,
@@ -190,7 +191,7 @@ struct PairArgs {
 // ring of 4 steps, 128 x 128 tiles 31.3 / 45.1 / 46.7 and 64 x 64 tiles 48.3 /
 // 38.9 / 23.2; three steps in flight 31.8 / 32.1 / 19.8.  One form for all
 // sizes also keeps an output's sums independent of M and N: rows and column
-// slices agree bitwise.
+// slices that take it (mg_pair_pays) agree bitwise.
 __global__ __launch_bounds__(256, 2) void k_pair_gemm(const PairArgs p) {
   constexpr int T = 64, KW = 4;
   __shared__ float4v part[KW][4][4][64];  // [wave][32 x 32 block][v / 4][lane]
@@ -332,9 +333,34 @@ size_t mg_pair_bytes(int64_t R, int64_t K) {
 // weight's own bytes (N >= 32 always), or a MiB, go into the images, whose rows are
 // padded to 64: a 1 x 2^20 weight of 4 MiB would take 256.
 bool mg_pair_keeps(int64_t N, int64_t K) {
-  return N > 0 && K > 0 && N < ((int64_t)1 << 22) && K < ((int64_t)1 << 18) &&
+  return N > 0 && K >= 192 && N < ((int64_t)1 << 22) && K < ((int64_t)1 << 18) &&
          (int64_t)mg_pair_bytes(64, K) <= MG_PAIR_CHUNK_BYTES &&
          (int64_t)mg_pair_bytes(N, K) <= 8 * N * K + (1 << 20);
+}
+
+// Where the pairs pay: the split of A (a launch, and 12 bytes of traffic per
+// element beside the 4 that fp32 products read) against products at two to three
+// times the rate.  us a call on fp32 MFMA / on pairs, rows x K -> N:
+// - Short sums do not: 1024 x 128 -> 1024 7.5 / 9.4, 4096 x 64 -> 4096 33 / 40.
+//   At K = 192 only few rows (64 -> 64 7.7 / 7.9; K = 224 to 256 0.97 to 0.9 of the
+//   time) and many outputs (4096 -> 1024 22.2 / 21.1, 8192 -> 768 0.80).
+// - Few rows are bound by the chain over K, which the pairs' four waves share,
+//   whatever N is: 1024 x 256 -> 1 9.1 / 9.1, 16 x 512 -> 64 14.7 / 8.8, 2048 x
+//   384 -> 64 12.9 / 12.1, 1024 x 8192 -> 64 0.74, 2048 x 8192 -> 64 1.46; 1536 x
+//   256 -> 512 1.12, -> 768 0.90.
+// - Many rows are bound by the traffic of A at few columns: 32768 x 1024 -> 64
+//   50 / 86, -> 128 88 / 98, -> 256 151 / 123, -> 1024 564 / 321; 8192 x 384 -> 128
+//   1.40, 8192 x 1024 -> 128 0.80, 16384 x 384 -> 128 1.16, -> 192 0.91; 8192 x 256 ->
+//   256 1.11, -> 384 0.99; 8192 x 4096 -> 128 1.53, -> 192 1.12, -> 256 0.90; 4096 x
+//   8192 -> 384 1.04, -> 512 0.87.
+// A column slice of a weight gives bitwise the whole one's columns where both are
+// on one side of these lines: up to 1024 rows they read rows and K only (K >= 256).
+bool mg_pair_pays(int64_t M, int64_t N, int64_t K) {
+  if (K < 256) return K >= 192 && (M <= 128 || (N >= 768 && M * N >= (int64_t)1 << 22));
+  if (M <= 2048 && M * K <= (int64_t)1 << 23 && K >= (M <= 1024 ? 256 : 384)) return true;
+  if (K < 384) return N >= (M <= 2048 ? 768 : 384);
+  if (K <= 2048) return N >= (M <= 8192 ? 128 : 192);
+  return K <= 4096 ? N >= 256 : K <= 8192 && N >= 512;
 }
 
 mg_status mg_pair_split(mg_ctx *ctx, const float *x_dev, int64_t R, int64_t K, void *img) {
@@ -346,10 +372,11 @@ mg_status mg_pair_split(mg_ctx *ctx, const float *x_dev, int64_t R, int64_t K, v
 #define MG_SPLIT(TPR, UL)                                                                    \
   hipLaunchKernelGGL((k_pair_split<TPR, UL>), dim3((unsigned)(rp / (256 / TPR))), dim3(256), 0, \
                      ctx->stream, x_dev, R, K, nk, vec, im, ex)
-  if (rp * K >= (int64_t)1 << 20 && K <= 2048) {
+  if (rp * K >= (int64_t)1 << 20 && (K <= 2048 || rp >= 2048)) {
     if (K <= 512) MG_SPLIT(32, 2);
     else if (K <= 1024) MG_SPLIT(32, 4);
-    else MG_SPLIT(32, 8);
+    else if (K <= 2048) MG_SPLIT(32, 8);
+    else MG_SPLIT(32, 0);
   } else {
     if (K <= 2048) MG_SPLIT(256, 1);
     else if (K <= 8192) MG_SPLIT(256, 4);

@@ -30,13 +30,14 @@ class Hip:
         return call
 
 
-SHAPES = dict(a=(100, 96), x=(2, 40, 9, 9), w=(24, 40, 3, 3), q=(1, 1, 256), k=(1, 1, 128),
+SHAPES = dict(a=(100, 320), x=(2, 40, 9, 9), w=(24, 40, 3, 3), q=(1, 1, 256), k=(1, 1, 128),
               v=(1, 1, 128), pk=(1, 2, 300, 64), pv=(1, 2, 300, 64))
 OUTPUTS = dict(gemm=(100, 70), conv=(2, 24, 9, 9), gqa=(1, 1, 256), ko=(1, 2, 301, 64),
                vo=(1, 2, 301, 64))
 
 
 def run(ops, ctx, d, fw, gemm_only):
+    # (a holds 100 rows of either K.)
     fw.gemm_dev(d["a"].ptr, 100, d["gemm"].ptr)
     if gemm_only:
         return
@@ -47,16 +48,17 @@ def run(ops, ctx, d, fw, gemm_only):
                                   past_value_ptr=d["pv"].ptr, past_len=300, ctx=ctx)
 
 
+@pytest.mark.parametrize("k", [96, 320])  # without and with digit pairs
 @pytest.mark.parametrize("warm", [True, False])
-def test_graph_replays(ops, warm):
+def test_graph_replays(ops, warm, k):
     rng = np.random.default_rng(1)
     ctx = ops.Context()
     hip = Hip()
     stream, graph, exe = C.c_void_p(), C.c_void_p(), C.c_void_p()
     hip.hipStreamCreate(C.byref(stream))
     ctx.set_stream(stream.value)
-    fw = ops.F32Weight(rng.standard_normal((70, 96)).astype(np.float32), trans_b=True, ctx=ctx)
-    big = ops.F32Weight(rng.standard_normal((64, 1024)).astype(np.float32), trans_b=True, ctx=ctx)
+    fw = ops.F32Weight(rng.standard_normal((70, k)).astype(np.float32), trans_b=True, ctx=ctx)
+    big = ops.F32Weight(rng.standard_normal((256, 1024)).astype(np.float32), trans_b=True, ctx=ctx)
     d = {key: ops.DeviceBuffer(4 * int(np.prod(s))) for key, s in {**SHAPES, **OUTPUTS}.items()}
 
     def fill(names):
@@ -88,10 +90,10 @@ def test_graph_replays(ops, warm):
         for key, want in results().items():
             if warm:
                 np.testing.assert_array_equal(got[key], want)
-            else:  # the graph holds the fp32 kernel: sums of 96 products, 2^-17 of ~40
+            else:  # the graph holds the fp32 kernel: sums of k products, 2^-19 of ~100
                 np.testing.assert_allclose(got[key], want, rtol=0, atol=1e-4)
         # A workspace larger than the graph's, other data in it.
-        a, z = ops.DeviceBuffer(4096 * step * 4096), ops.DeviceBuffer(4096 * step * 256)
+        a, z = ops.DeviceBuffer(4096 * step * 4096), ops.DeviceBuffer(4096 * step * 1024)
         big.gemm_dev(a.ptr, 4096 * step, z.ptr)
         hip.hipStreamSynchronize(stream)
         a.free()

@@ -30,7 +30,16 @@ def check(y, a, w, c=0.0, alpha=1.0, beta=1.0):
 
 @pytest.mark.parametrize("m,k,n", [(1, 1, 1), (63, 15, 65), (65, 64, 63), (64, 65, 64),
                                    (1, 2049, 130), (130, 8200, 70), (2049, 513, 65),
-                                   (1030, 1025, 33), (700, 1537, 129), (4096, 384, 200)])
+                                   (1030, 1025, 33), (700, 1537, 129), (4096, 384, 200),
+                                   # The sizes that take pairs, to either side of each line.
+                                   (1, 256, 1), (63, 257, 65), (65, 319, 63), (64, 320, 64),
+                                   (128, 192, 64), (129, 192, 64), (64, 191, 64), (700, 200, 6000),
+                                   (690, 200, 6000), (1024, 256, 3), (1025, 257, 66),
+                                   (1030, 260, 767), (1030, 260, 768), (2049, 260, 383),
+                                   (2049, 260, 384), (1025, 384, 65), (2049, 384, 128),
+                                   (2049, 513, 127), (8193, 384, 191), (8193, 385, 192),
+                                   (2050, 4100, 255), (2050, 4096, 255), (2050, 4096, 256),
+                                   (2050, 4100, 511), (2050, 4100, 512), (30, 9000, 65)])
 def test_tile_edges(ops, m, k, n):
     rng = np.random.default_rng(m + k + n)
     a = rng.standard_normal((m, k)).astype(np.float32)
