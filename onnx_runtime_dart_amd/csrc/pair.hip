@@ -32,7 +32,7 @@ namespace {
 // TPR UL), UL = 0 reads the row twice.  Bound by memory at large R (4096 x 1536:
 // 25 MB in, 25 MB out, 10.4 us, 4.8 TB/s) and by its launch and one round trip at small ones, so
 // rows of few workgroups take a whole workgroup each (long rows in eights, whose
-// pieces fill whole lines: a call of 4096 x 4096 -> 1024 0.7 of the time).
+// pieces fill whole lines: 4096 x 4096 -> 512 140 -> 115 us a call).
 template <int TPR, int UL>
 __global__ __launch_bounds__(256) void k_pair_split(const float *__restrict__ X, int64_t R,
                                                     int64_t K, int nk, int vec,
