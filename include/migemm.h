@@ -76,7 +76,8 @@ mg_status mg_ctx_destroy(mg_ctx *ctx);
 
 /* Uses `hip_stream` (a hipStream_t, may be NULL for the null stream) for all
  * later work of the context instead of its own stream.  The caller keeps
- * ownership of the stream. */
+ * ownership of the stream.  Waits for the work on the stream used so far, which
+ * may still use the context's workspace. */
 mg_status mg_ctx_set_stream(mg_ctx *ctx, void *hip_stream);
 /* The hipStream_t the context launches on. */
 mg_status mg_ctx_get_stream(mg_ctx *ctx, void **hip_stream);

@@ -288,7 +288,9 @@ mg_status mg_ctx_destroy(mg_ctx *ctx) {
 mg_status mg_ctx_set_stream(mg_ctx *ctx, void *hip_stream) {
   if (!ctx) return mg_fail(MG_INVALID_ARGUMENT, "mg_ctx_set_stream: null context");
   MG_TRY(mg_use_device(ctx));
-  if (ctx->stream) MG_HIP(hipStreamSynchronize(ctx->stream));
+  // The workspace changes streams: the old stream's calls, the null stream's too,
+  // are done with it first.  (Allowed while the new stream is capturing.)
+  if (ctx->stream || hip_stream) MG_HIP(hipStreamSynchronize(ctx->stream));
   if (ctx->own_stream && ctx->stream) MG_HIP(hipStreamDestroy(ctx->stream));
   ctx->stream = static_cast<hipStream_t>(hip_stream);
   ctx->own_stream = false;

@@ -1,6 +1,7 @@
 """Ops with an optional workspace under HIP graph capture: replays give the
 eager results, also after the workspace has grown past the captured one, and a
-Gemm captured without any workspace runs the kernel that needs none."""
+Gemm captured without any workspace runs the kernel that needs none.  The
+workspace when the context changes streams."""
 import ctypes as C
 
 import numpy as np
@@ -104,5 +105,56 @@ def test_graph_replays(ops, warm, k):
         b.free()
     fw.release()
     big.release()
+    ctx.close()
+    hip.hipStreamDestroy(stream)
+
+
+@pytest.mark.parametrize("flags", [0, 1])  # blocking, non-blocking with the null stream
+def test_stream_switch(ops, flags):
+    # Calls pending on the null stream keep the workspace to themselves: the
+    # switch to another stream, also one that is capturing, waits for them.
+    rng = np.random.default_rng(2)
+    hip = Hip()
+    ctx = ops.Context()
+    ctx.set_stream(0)
+    m, k, n = 4096, 1536, 384
+    w = ops.F32Weight(rng.standard_normal((n, k)).astype(np.float32), trans_b=True, ctx=ctx)
+    a = [ops.DeviceBuffer.from_array(rng.standard_normal((m, k)).astype(np.float32), ctx)
+         for _ in range(2)]
+    y = [ops.DeviceBuffer(m * n * 4, ctx) for _ in range(8)]
+
+    def result(b):
+        return b.to_array((m, n), np.float32)
+
+    w.gemm_dev(a[0].ptr, m, y[6].ptr)
+    w.gemm_dev(a[1].ptr, m, y[7].ptr)
+    want = [result(b) for b in y[6:]]
+    stream, graph, exe = C.c_void_p(), C.c_void_p(), C.c_void_p()
+    hip.hipStreamCreateWithFlags(C.byref(stream), flags)
+    for b in y[:5]:
+        w.gemm_dev(a[0].ptr, m, b.ptr)
+    ctx.set_stream(stream.value)
+    w.gemm_dev(a[1].ptr, m, y[5].ptr)
+    np.testing.assert_array_equal(result(y[5]), want[1])
+    ctx.set_stream(0)
+    for b in y[:5]:
+        np.testing.assert_array_equal(result(b), want[0])
+        w.gemm_dev(a[0].ptr, m, b.ptr)
+    hip.hipStreamBeginCapture(stream, 0)
+    ctx.set_stream(stream.value)
+    w.gemm_dev(a[1].ptr, m, y[5].ptr)
+    hip.hipStreamEndCapture(stream, C.byref(graph))
+    hip.hipGraphInstantiate(C.byref(exe), graph, None, None, C.c_size_t(0))
+    for _ in range(3):
+        w.gemm_dev(a[0].ptr, m, y[5].ptr)
+        hip.hipGraphLaunch(exe, stream)
+        np.testing.assert_array_equal(result(y[5]), want[1])
+    for b in y[:5]:
+        np.testing.assert_array_equal(result(b), want[0])
+    hip.hipGraphExecDestroy(exe)
+    hip.hipGraphDestroy(graph)
+    for b in a + y:
+        b.free()
+    w.release()
     ctx.close()
     hip.hipStreamDestroy(stream)
