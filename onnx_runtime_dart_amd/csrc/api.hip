@@ -155,12 +155,25 @@ hipEvent_t prof_event(mg_ctx *ctx) {
   return e;
 }
 
+namespace {
+bool capturing(const mg_ctx *ctx) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(ctx->stream, &st) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;
+  }
+  return st != hipStreamCaptureStatusNone;
+}
+}  // namespace
+
 mg_status mg_ws_reserve(mg_ctx *ctx, size_t bytes) {
-  if (bytes <= ctx->ws_bytes) return MG_OK;
+  if (bytes <= ctx->ws_bytes) {
+    if (bytes && !ctx->ws_captured) ctx->ws_captured = capturing(ctx);
+    return MG_OK;
+  }
   if (ctx->ws) {
     if (ctx->ws_captured) {
       ctx->ws_old.push_back(ctx->ws);
-      ctx->ws_captured = false;
     } else {
       MG_HIP(hipStreamSynchronize(ctx->stream));
       MG_HIP(hipFree(ctx->ws));
@@ -171,21 +184,13 @@ mg_status mg_ws_reserve(mg_ctx *ctx, size_t bytes) {
   const size_t want = mg_align(bytes, 1 << 20);
   MG_HIP(hipMalloc(&ctx->ws, want));
   ctx->ws_bytes = want;
+  ctx->ws_captured = capturing(ctx);
   return MG_OK;
 }
 
 bool mg_ws_optional(mg_ctx *ctx, size_t bytes) {
   if (ctx->max_bytes >= 0 && (int64_t)bytes > ctx->max_bytes) return false;
-  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(ctx->stream, &st) != hipSuccess) {
-    (void)hipGetLastError();
-    st = hipStreamCaptureStatusActive;
-  }
-  if (st != hipStreamCaptureStatusNone) {
-    if (bytes > ctx->ws_bytes) return false;
-    ctx->ws_captured = true;
-    return true;
-  }
+  if (bytes > ctx->ws_bytes && capturing(ctx)) return false;
   if (mg_ws_reserve(ctx, bytes) == MG_OK) return true;
   g_last_error.clear();
   (void)hipGetLastError();

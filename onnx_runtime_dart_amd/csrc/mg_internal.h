@@ -56,8 +56,9 @@ struct mg_ctx {
   // host-pointer calls.  Reused across calls of this context only.
   void *ws = nullptr;
   size_t ws_bytes = 0;
-  // A captured graph may hold the address of ws (mg_ws_optional): a larger
-  // workspace then does not free it; it waits in ws_old for the context's end.
+  // A captured graph may hold the address of ws (a call reserved it while the
+  // stream was capturing): a larger workspace then does not free it; it waits in
+  // ws_old for the context's end.
   bool ws_captured = false;
   std::vector<void *> ws_old;
   // Compute units of the device (grid sizing).
@@ -157,7 +158,7 @@ mg_status mg_ws_reserve(mg_ctx *ctx, size_t bytes);
 // Whether an op that can also run with less (or no) workspace may take
 // `bytes` of it: within the byte budget, and there or allocated now.  Under
 // stream capture only a workspace that is already large enough serves (no
-// allocation there), and it then outlives growth for the graph's sake.
+// allocation there).
 bool mg_ws_optional(mg_ctx *ctx, size_t bytes);
 // Sets the context's device current on this thread.
 mg_status mg_use_device(mg_ctx *ctx);

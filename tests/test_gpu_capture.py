@@ -109,6 +109,48 @@ def test_graph_replays(ops, warm, k):
     hip.hipStreamDestroy(stream)
 
 
+def test_any_captured_workspace_outlives_growth(ops):
+    # A graph of an op that cannot do without its workspace (a decode GEMV split
+    # over K); later calls need a larger one.
+    rng = np.random.default_rng(3)
+    hip = Hip()
+    ctx = ops.Context()
+    stream, graph, exe = C.c_void_p(), C.c_void_p(), C.c_void_p()
+    hip.hipStreamCreate(C.byref(stream))
+    ctx.set_stream(stream.value)
+    k, n, bs = 8192, 2048, 32
+    w = ops.NBitsWeight(rng.integers(0, 256, (n, k // bs, bs // 2), dtype=np.uint8),
+                        rng.uniform(0.002, 0.02, (n, k // bs)).astype(np.float32), None, k=k, n=n,
+                        block_size=bs, ctx=ctx)
+    big = ops.F32Weight(rng.standard_normal((256, 1024)).astype(np.float32), trans_b=True, ctx=ctx)
+    a = ops.DeviceBuffer.from_array(rng.standard_normal((1, k)).astype(np.float32), ctx)
+    y = ops.DeviceBuffer(n * 4, ctx)
+    w.run_dev(a.ptr, 1, y.ptr)
+    want = y.to_array((n,), np.float32)
+    hip.hipStreamBeginCapture(stream, 0)
+    w.run_dev(a.ptr, 1, y.ptr)
+    hip.hipStreamEndCapture(stream, C.byref(graph))
+    hip.hipGraphInstantiate(C.byref(exe), graph, None, None, C.c_size_t(0))
+    zero = np.zeros(n, np.float32)
+    for step in (1, 2, 3):
+        rows = 4096 * step
+        x, z = ops.DeviceBuffer(4096 * rows, ctx), ops.DeviceBuffer(1024 * rows, ctx)
+        big.gemm_dev(x.ptr, rows, z.ptr)
+        x.free()
+        z.free()
+        ops.check(ops.lib.mg_buffer_upload(ctx.handle, y.ptr, zero.ctypes.data, zero.nbytes))
+        hip.hipGraphLaunch(exe, stream)
+        np.testing.assert_array_equal(y.to_array((n,), np.float32), want)
+    hip.hipGraphExecDestroy(exe)
+    hip.hipGraphDestroy(graph)
+    for b in (a, y):
+        b.free()
+    w.release()
+    big.release()
+    ctx.close()
+    hip.hipStreamDestroy(stream)
+
+
 @pytest.mark.parametrize("flags", [0, 1])  # blocking, non-blocking with the null stream
 def test_stream_switch(ops, flags):
     # Calls pending on the null stream keep the workspace to themselves: the
