@@ -155,8 +155,7 @@ hipEvent_t prof_event(mg_ctx *ctx) {
   return e;
 }
 
-namespace {
-bool capturing(const mg_ctx *ctx) {
+bool mg_capturing(const mg_ctx *ctx) {
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(ctx->stream, &st) != hipSuccess) {
     (void)hipGetLastError();
@@ -164,11 +163,10 @@ bool capturing(const mg_ctx *ctx) {
   }
   return st != hipStreamCaptureStatusNone;
 }
-}  // namespace
 
 mg_status mg_ws_reserve(mg_ctx *ctx, size_t bytes) {
   if (bytes <= ctx->ws_bytes) {
-    if (bytes && !ctx->ws_captured) ctx->ws_captured = capturing(ctx);
+    if (bytes && !ctx->ws_captured) ctx->ws_captured = mg_capturing(ctx);
     return MG_OK;
   }
   if (ctx->ws) {
@@ -184,13 +182,13 @@ mg_status mg_ws_reserve(mg_ctx *ctx, size_t bytes) {
   const size_t want = mg_align(bytes, 1 << 20);
   MG_HIP(hipMalloc(&ctx->ws, want));
   ctx->ws_bytes = want;
-  ctx->ws_captured = capturing(ctx);
+  ctx->ws_captured = mg_capturing(ctx);
   return MG_OK;
 }
 
 bool mg_ws_optional(mg_ctx *ctx, size_t bytes) {
   if (ctx->max_bytes >= 0 && (int64_t)bytes > ctx->max_bytes) return false;
-  if (bytes > ctx->ws_bytes && capturing(ctx)) return false;
+  if (bytes > ctx->ws_bytes && mg_capturing(ctx)) return false;
   if (mg_ws_reserve(ctx, bytes) == MG_OK) return true;
   g_last_error.clear();
   (void)hipGetLastError();
@@ -658,7 +656,7 @@ mg_status mg_matmul_nbits_dev_noalloc(mg_ctx *ctx, const mg_weight *w, const flo
   if (M < 0) return mg_fail(MG_INVALID_ARGUMENT, "MatMulNBits: invalid K, N, block_size or input shape");
   if (M == 0) return MG_OK;
   if (!a_dev || !y_dev) return mg_fail(MG_INVALID_ARGUMENT, "mg_matmul_nbits: null buffer");
-  const size_t ws = mg_nbits_ws_bytes(ctx, w, M);
+  const size_t ws = mg_nbits_ws_bytes(ctx, w, M, MG_NBITS_SCRATCH);
   if (ws > (size_t)MG_NOALLOC_SCRATCH_BYTES)
     return mg_fail(MG_INVALID_ARGUMENT,
                    "mg_matmul_nbits_dev_noalloc: " + std::to_string(M) + " rows need " +
@@ -668,7 +666,7 @@ mg_status mg_matmul_nbits_dev_noalloc(mg_ctx *ctx, const mg_weight *w, const flo
   MG_TRY(mg_check_control(ctx, 0));
   void *s = scratch_dev(ctx->device);
   if (!s) return mg_fail(MG_DEVICE_ERROR, "mg_matmul_nbits_dev_noalloc: no scratch on this device");
-  return mg_nbits_run(ctx, w, a_dev, M, y_dev, s);
+  return mg_nbits_run(ctx, w, a_dev, M, y_dev, s, MG_NBITS_SCRATCH);
 }
 
 namespace {
@@ -730,13 +728,14 @@ mg_status mg_matmul_nbits(mg_ctx *ctx, const mg_weight *w, const float *a, int64
   Staging s;
   const size_t oa = s.take((size_t)(M * w->K) * 4);
   const size_t oy = s.take((size_t)(M * w->N) * 4);
-  const size_t ow = s.take(mg_nbits_ws_bytes(ctx, w, M));
+  const int64_t staged = (int64_t)s.off;
+  const size_t ow = s.take(mg_nbits_ws_bytes(ctx, w, M, staged));
   MG_TRY(mg_check_control(ctx, (int64_t)s.off));
   MG_TRY(mg_ws_reserve(ctx, s.off));
   char *base = static_cast<char *>(ctx->ws);
   MG_HIP(hipMemcpyAsync(base + oa, a, (size_t)(M * w->K) * 4, hipMemcpyHostToDevice, ctx->stream));
   MG_TRY(mg_nbits_run(ctx, w, reinterpret_cast<float *>(base + oa), M,
-                      reinterpret_cast<float *>(base + oy), base + ow));
+                      reinterpret_cast<float *>(base + oy), base + ow, staged));
   MG_HIP(hipMemcpyAsync(y, base + oy, (size_t)(M * w->N) * 4, hipMemcpyDeviceToHost, ctx->stream));
   MG_HIP(hipStreamSynchronize(ctx->stream));
   return MG_OK;

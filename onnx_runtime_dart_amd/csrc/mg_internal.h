@@ -160,6 +160,8 @@ mg_status mg_ws_reserve(mg_ctx *ctx, size_t bytes);
 // stream capture only a workspace that is already large enough serves (no
 // allocation there).
 bool mg_ws_optional(mg_ctx *ctx, size_t bytes);
+// Whether the context's stream is capturing (or cannot be asked).
+bool mg_capturing(const mg_ctx *ctx);
 // Sets the context's device current on this thread.
 mg_status mg_use_device(mg_ctx *ctx);
 // Copies `bytes` of host memory to device memory on the context's stream.
@@ -194,11 +196,16 @@ void mg_nbits_free(mg_weight *w);
 // of its images (allocates w->nbits.img; synchronous).
 bool mg_nbits_f8_eligible(const mg_nbits_dev &d);
 mg_status mg_nbits_f8_images(mg_ctx *ctx, mg_weight *w);
-// Workspace bytes mg_nbits_run needs for M rows.
-size_t mg_nbits_ws_bytes(const mg_ctx *ctx, const mg_weight *w, int64_t M);
-// a_dev [M, K] f32, y_dev [M, N] f32; ws holds mg_nbits_ws_bytes bytes.
+// Workspace bytes mg_nbits_run needs for M rows, the plan's choice of them
+// included: `staged` are the bytes that the call takes of the context's workspace
+// (and of its byte budget) beside them, or MG_NBITS_SCRATCH for the
+// allocation-free entry point's own scratch.
+constexpr int64_t MG_NBITS_SCRATCH = -1;
+size_t mg_nbits_ws_bytes(const mg_ctx *ctx, const mg_weight *w, int64_t M, int64_t staged = 0);
+// a_dev [M, K] f32, y_dev [M, N] f32; ws holds mg_nbits_ws_bytes bytes (of the
+// same `staged`).
 mg_status mg_nbits_run(mg_ctx *ctx, const mg_weight *w, const float *a_dev,
-                       int64_t M, float *y_dev, void *ws);
+                       int64_t M, float *y_dev, void *ws, int64_t staged = 0);
 // n <= 4 weights with the same K, block size and zero-point kind applied to
 // one activation a_dev: y_dev[i] = a . W_i^T.  Decode shapes run as one
 // launch; ws holds mg_nbits_group_ws_bytes bytes.
@@ -209,7 +216,7 @@ size_t mg_nbits_group_ws_bytes(const mg_ctx *ctx, int n, const mg_weight *const 
 // the 3..16-row GEMV it replaces the activation prepass.
 mg_status mg_nbits_run_group(mg_ctx *ctx, int n, const mg_weight *const *w,
                              const float *a_dev, int64_t M, float *const *y_dev, void *ws,
-                             const void *split = nullptr);
+                             const void *split = nullptr, int64_t staged = 0);
 // K padded as a MatMulNBits weight of this block size pads it (the split
 // activation buffer covers k < kpad).
 inline int64_t mg_nbits_kpad(int64_t K, int64_t bs) {

@@ -1663,18 +1663,22 @@ NbitsPlan plan_nbits_ws(const mg_ctx *ctx, const mg_weight *w, int64_t M, int64_
   return p;
 }
 
-// The wide plan where its workspace is within the context's byte budget and
-// within what the allocation-free entry point has (or no larger than the
-// other plan's): no call is refused for the sake of a split.
+// The wide plan where its workspace is no larger than the other plan's, or can be
+// had: within 32 MiB (what the allocation-free entry point has), within the
+// context's byte budget beside the call's `staged` bytes, and under stream capture
+// within the workspace that is there.  No call is refused for the sake of a split.
 NbitsPlan plan_nbits(const mg_ctx *ctx, const mg_weight *w, int64_t M, int64_t ng_total,
-                     int64_t n_total, bool imgs) {
+                     int64_t n_total, bool imgs, int64_t staged) {
   const NbitsPlan p = plan_nbits_ws(ctx, w, M, ng_total, n_total, imgs, true);
   if (p.path != 1) return p;
   const NbitsPlan q = plan_nbits_ws(ctx, w, M, ng_total, n_total, imgs, false);
-  const size_t lim = ctx->max_bytes >= 0
-                         ? std::min<size_t>(MG_NOALLOC_SCRATCH_BYTES, (size_t)ctx->max_bytes)
-                         : MG_NOALLOC_SCRATCH_BYTES;
-  return p.total <= std::max(q.total, lim) ? p : q;
+  if (p.total <= q.total) return p;
+  if (p.total > (size_t)MG_NOALLOC_SCRATCH_BYTES) return q;
+  if (staged == MG_NBITS_SCRATCH) return p;
+  const int64_t all = staged + (int64_t)p.total;
+  if (ctx->max_bytes >= 0 && all > ctx->max_bytes) return q;
+  if ((size_t)all > ctx->ws_bytes && mg_capturing(ctx)) return q;
+  return p;
 }
 
 GemvSet make_set(int n, const mg_weight *const *w, float *const *y) {
@@ -2044,14 +2048,15 @@ void mg_nbits_free(mg_weight *w) {
   d = mg_nbits_dev{};
 }
 
-size_t mg_nbits_ws_bytes(const mg_ctx *ctx, const mg_weight *w, int64_t M) {
-  return plan_nbits(ctx, w, M, w->nbits.ng, w->N, w->nbits.img != nullptr).total;
+size_t mg_nbits_ws_bytes(const mg_ctx *ctx, const mg_weight *w, int64_t M, int64_t staged) {
+  return plan_nbits(ctx, w, M, w->nbits.ng, w->N, w->nbits.img != nullptr, staged).total;
 }
 
 namespace {
 // The plan of a group of weights launched together: member 0's kind of path,
 // sized for all members.
-NbitsPlan plan_group(const mg_ctx *ctx, int n, const mg_weight *const *w, int64_t M) {
+NbitsPlan plan_group(const mg_ctx *ctx, int n, const mg_weight *const *w, int64_t M,
+                     int64_t staged) {
   int64_t ng = 0, nn = 0;
   bool imgs = true;  // every member has prefill images
   for (int i = 0; i < n; i++) {
@@ -2059,13 +2064,13 @@ NbitsPlan plan_group(const mg_ctx *ctx, int n, const mg_weight *const *w, int64_
     nn += w[i]->N;
     imgs = imgs && w[i]->nbits.img != nullptr;
   }
-  return plan_nbits(ctx, w[0], M, ng, nn, imgs);
+  return plan_nbits(ctx, w[0], M, ng, nn, imgs, staged);
 }
 }  // namespace
 
 size_t mg_nbits_group_ws_bytes(const mg_ctx *ctx, int n, const mg_weight *const *w,
                                int64_t M) {
-  return plan_group(ctx, n, w, M).total;
+  return plan_group(ctx, n, w, M, 0).total;
 }
 
 namespace {
@@ -2077,13 +2082,13 @@ mg_status prefill_run(mg_ctx *ctx, int n, const mg_weight *const *w, const float
 
 mg_status mg_nbits_run_group(mg_ctx *ctx, int n, const mg_weight *const *w,
                              const float *a_dev, int64_t M, float *const *y_dev, void *ws,
-                             const void *split) {
+                             const void *split, int64_t staged) {
   if (M == 0 || n == 0) return MG_OK;
   int64_t ng = 0;
   for (int i = 0; i < n; i++) ng += w[i]->nbits.ng;
   const mg_weight *w0 = w[0];
   const mg_nbits_dev &d = w0->nbits;
-  const NbitsPlan p = plan_group(ctx, n, w, M);
+  const NbitsPlan p = plan_group(ctx, n, w, M, staged);
   hipStream_t st = ctx->stream;
   char *base = static_cast<char *>(ws);
   if (p.path == 0) {
@@ -2207,8 +2212,8 @@ mg_status mg_nbits_run_group(mg_ctx *ctx, int n, const mg_weight *const *w,
 }
 
 mg_status mg_nbits_run(mg_ctx *ctx, const mg_weight *w, const float *a_dev,
-                       int64_t M, float *y_dev, void *ws) {
-  return mg_nbits_run_group(ctx, 1, &w, a_dev, M, &y_dev, ws);
+                       int64_t M, float *y_dev, void *ws, int64_t staged) {
+  return mg_nbits_run_group(ctx, 1, &w, a_dev, M, &y_dev, ws, nullptr, staged);
 }
 
 namespace {

@@ -18,12 +18,12 @@ def ops():
     return _ops
 
 
-def weight(ops, rng, k, n, bs):
+def weight(ops, rng, k, n, bs, ctx=None):
     nb = -(-k // bs)
     b = rng.integers(0, 256, (n, nb, bs // 2), dtype=np.uint8)
     s = rng.uniform(0.002, 0.02, (n, nb)).astype(np.float32)
     zp = rng.integers(0, 256, (n, (nb + 1) // 2), dtype=np.uint8)
-    return (b, s, zp), ops.NBitsWeight(b, s, zp, k=k, n=n, block_size=bs)
+    return (b, s, zp), ops.NBitsWeight(b, s, zp, k=k, n=n, block_size=bs, ctx=ctx)
 
 
 def check(y, a, w, k, bs):
@@ -68,3 +68,58 @@ def test_plan_under_a_byte_budget(ops):
     for d in (ad, yd):
         d.free()
     h.release()
+
+
+def test_host_call_under_a_byte_budget(ops):
+    # The activations and results staged by the host entry point count against
+    # the budget too: 7.4 MB beside 26 MB of the wide plan or 11 of the other.
+    rng = np.random.default_rng(8)
+    m, k, n, bs = 301, 4096, 2048, 32
+    w, h = weight(ops, rng, k, n, bs)
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    ctx = ops.default_context()
+    ctx.set_control(None, max_bytes=27 << 20)
+    try:
+        y = h(a)
+    finally:
+        ctx.set_control(None, max_bytes=-1)
+    check(y, a, w, k, bs)
+    h.release()
+
+
+def test_plan_under_capture(ops):
+    # A capturing stream cannot grow the workspace: the plan keeps to the one
+    # that an earlier call left (here under a byte budget), and replays give what
+    # that call gave, also after the wide plan has run beside them.
+    import ctypes as C
+    from test_gpu_capture import Hip
+    hip, ctx = Hip(), ops.Context()
+    stream, graph, exe = C.c_void_p(), C.c_void_p(), C.c_void_p()
+    hip.hipStreamCreate(C.byref(stream))
+    ctx.set_stream(stream.value)
+    rng = np.random.default_rng(9)
+    m, k, n, bs = 301, 4096, 2048, 32
+    w, h = weight(ops, rng, k, n, bs, ctx)
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    ad, yd = ops.DeviceBuffer.from_array(a, ctx), ops.DeviceBuffer(m * n * 4, ctx)
+    ctx.set_control(None, max_bytes=12 << 20)
+    h.run_dev(ad.ptr, m, yd.ptr)
+    ctx.set_control(None, max_bytes=-1)
+    eager = yd.to_array((m, n), np.float32)
+    check(eager, a, w, k, bs)
+    hip.hipStreamBeginCapture(stream, 0)
+    h.run_dev(ad.ptr, m, yd.ptr)
+    hip.hipStreamEndCapture(stream, C.byref(graph))
+    hip.hipGraphInstantiate(C.byref(exe), graph, None, None, C.c_size_t(0))
+    for _ in range(3):
+        h.run_dev(ad.ptr, m, yd.ptr)
+        check(yd.to_array((m, n), np.float32), a, w, k, bs)
+        hip.hipGraphLaunch(exe, stream)
+        np.testing.assert_array_equal(yd.to_array((m, n), np.float32), eager)
+    hip.hipGraphExecDestroy(exe)
+    hip.hipGraphDestroy(graph)
+    for d in (ad, yd):
+        d.free()
+    h.release()
+    ctx.close()
+    hip.hipStreamDestroy(stream)
