@@ -106,7 +106,12 @@ mg_status mg_ctx_profile_clear(mg_ctx *ctx);
  * block sizes >= 128 have images.  No counterpart in the reference, which
  * dequantises the weight to fp32 on every call
  * (lib/src/onnx_qlinear_ops.dart:208-226); for callers that run only decode
- * rows and want the smaller footprint. */
+ * rows and want the smaller footprint.
+ *
+ * The same for the fp16 digit pairs of fp32 operators: with images disabled,
+ * fp32 weights created from now on keep no pairs (4 bytes per element less), and
+ * Conv and Gemm form their products in fp32, exact operands and no workspace for
+ * digits. */
 mg_status mg_ctx_set_prefill_images(mg_ctx *ctx, int32_t enable);
 
 /* Cooperative cancellation and byte budget, checked before every launch

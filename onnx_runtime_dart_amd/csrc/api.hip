@@ -610,7 +610,7 @@ mg_status mg_weight_f32_create(mg_ctx *ctx, const float *b, int64_t rows, int64_
   }
   // Its pair images; a weight without them (or no memory left) runs on the fp32
   // MFMA kernel.
-  if (mg_pair_keeps(N, K)) {
+  if (ctx->prefill_images && mg_pair_keeps(N, K)) {
     const size_t pb = mg_pair_bytes(N, K);
     if (hipMalloc(&w->f32.pair, pb) != hipSuccess) {
       w->f32.pair = nullptr;
@@ -1962,7 +1962,7 @@ mg_status conv_host(mg_ctx *ctx, mg_conv_problem p, const void *x, size_t x_el, 
   const size_t ox = s.take((size_t)nx * x_el), ow = s.take((size_t)nw * w_el),
                ob = s.take(bias ? bias_bytes : 0), oy = s.take((size_t)ny * y_el),
                oz = s.take(wz.size() * 4), om = s.take(mult.size() * 8);
-  const size_t pb = mg_conv_pair_bytes(p);
+  const size_t pb = ctx->prefill_images ? mg_conv_pair_bytes(p) : 0;
   const bool pair = pb && mg_ws_optional(ctx, s.off + mg_align(pb));
   const size_t oph = s.take(pair ? pb : mg_conv_ws_bytes(p));
   MG_TRY(mg_check_control(ctx, (int64_t)s.off));
@@ -1990,7 +1990,7 @@ mg_status conv_dev(mg_ctx *ctx, mg_conv_problem p, const void *x, const void *w,
   MG_TRY(mg_use_device(ctx));
   Staging s;
   const size_t oz = s.take(wz.size() * 4), om = s.take(mult.size() * 8);
-  const size_t pb = mg_conv_pair_bytes(p);
+  const size_t pb = ctx->prefill_images ? mg_conv_pair_bytes(p) : 0;
   const bool pair = pb && mg_ws_optional(ctx, s.off + mg_align(pb));
   const size_t oph = s.take(pair ? pb : mg_conv_ws_bytes(p));
   MG_TRY(mg_check_control(ctx, (int64_t)s.off));

@@ -71,8 +71,8 @@ struct mg_ctx {
   bool prof = false;
   std::vector<mg_prof_rec> prof_recs;
   std::vector<hipEvent_t> prof_pool;
-  // MatMulNBits weights created afterwards keep their prefill images
-  // (mg_ctx_set_prefill_images).
+  // MatMulNBits and fp32 weights created afterwards keep their prefill and pair
+  // images, and fp32 Conv makes its own (mg_ctx_set_prefill_images).
   bool prefill_images = true;
   // The two chunk slots of the MatMulNBits upload (pinned host and device,
   // up_slot bytes each, grow-only), held until the context is destroyed so

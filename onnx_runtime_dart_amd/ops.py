@@ -93,7 +93,8 @@ class Context:
         calls on weights with images run the fp6 GEMM, those without the fp8
         GEMM that dequantises each tile (or the fp32 path for float zero
         points).  Both meet the MatMulNBits tolerance; the results differ in
-        rounding."""
+        rounding.  Disabled, fp32 weights created from now on keep no fp16
+        digit pairs, and Gemm on them and Conv form their products in fp32."""
         check(lib.mg_ctx_set_prefill_images(self.handle, int(bool(enable))))
 
     def profile_records(self) -> list:

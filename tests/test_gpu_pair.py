@@ -218,3 +218,30 @@ def test_inf_and_nan_beside_small(ops):
         np.testing.assert_array_equal(z[:, cols], clean[:, cols])
         np.testing.assert_array_equal(z[:, 11], a[:, 2] * np.float32(np.inf))
     assert np.isnan(z[:, 64]).all()
+
+
+def test_without_images(ops):
+    # A context with images disabled: no pairs, products of the operands as they
+    # are, so that a permutation and a filter of one tap copy bit for bit.
+    rng = np.random.default_rng(10)
+    k = 320
+    a = rng.standard_normal((70, k)).astype(np.float32)
+    order = rng.permutation(k)
+    w = np.eye(k, dtype=np.float32)[order]
+    x = rng.standard_normal((2, 32, 9, 9)).astype(np.float32)
+    v = np.zeros((32, 32, 3, 3), np.float32)
+    v[np.arange(32), order[order < 32], 1, 1] = 1
+    ctx = ops.default_context()
+    ctx.set_prefill_images(False)
+    try:
+        fw = ops.F32Weight(w, trans_b=True, ctx=ctx)
+        y = ops.op_conv(x, v, None, pads=[1] * 4)
+    finally:
+        ctx.set_prefill_images(True)
+    assert fw.info()[2] == 4 * k * k
+    np.testing.assert_array_equal(fw.gemm(a), a[:, order])
+    np.testing.assert_array_equal(y, x[:, order[order < 32]])
+    fw.release()
+    fw = ops.F32Weight(w, trans_b=True, ctx=ctx)
+    assert fw.info()[2] > 8 * k * k
+    fw.release()
