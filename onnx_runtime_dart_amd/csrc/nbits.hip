@@ -64,22 +64,26 @@ namespace {
 // ahl[((m32 * c4n + kg) * 8 + st) * 128 + 32 h + r] holds the hi fp16 x 8 of
 // row r, k = 128 kg + 16 st + 8 h .. +7, and +64 the lo part; texp[row] = e.
 // Rows past M and k past K are zeros.  Non-finite values pass through in hi.
-// Workgroup: one row, so that a few hundred rows reach every CU, neighbouring
-// rows (whose 16-byte pieces share lines) on one XCD.  Bound by the CUs' rate:
-// 301 rows of 8192 k took 16 us on 96 workgroups with a wave a row, 12.4 with
-// the row kept in registers, 15.7 on 48 of 8 rows that fill whole lines, 10.1 so.
-// UL > 0: a row has at most 256 UL 16-k pieces, and each lane reads its UL
+// TPR threads per row.  256: a workgroup per row, so that a few hundred rows
+// reach every CU, neighbouring rows (whose 16-byte pieces share lines) on one XCD.
+// Bound by the CUs' rate: 301 rows of 8192 k took 16 us on 96 workgroups with a
+// wave a row, 12.4 with the row kept in registers, 15.7 on 48 of 8 rows that fill
+// whole lines, 10.1 so.  64: four rows, for many short ones, which would leave most
+// of a workgroup idle (calls of 4096 x 128 -> 64 15.2 -> 13.1 us, 4096 x 512 25.3 ->
+// 23.6; at 1024 k no difference), and for row counts that would exceed a grid.
+// UL > 0: a row has at most TPR UL 16-k pieces, and each lane reads its UL
 // pieces once, with all loads in flight together, and keeps them in registers
 // for the split; UL = 0 (longer rows) reads the row twice.
-template <int UL>
+template <int TPR, int UL>
 __global__ __launch_bounds__(256) void k_af16split(
     const float *__restrict__ a, int64_t M, int64_t K, int c4n, int vec,
     uint4 *__restrict__ ahl, int *__restrict__ texp) {
   const int t = threadIdx.x;
-  constexpr int TPR = 256;
-  const int u0 = t;
-  // (The grid is the padded rows, a multiple of 128.)
-  const int64_t row = (int64_t)(blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  const int u0 = t % TPR;
+  // (The padded rows are a multiple of 128.)
+  const int64_t row = TPR == 256
+                          ? (int64_t)(blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3)
+                          : (int64_t)blockIdx.x * (256 / TPR) + t / TPR;
   const int64_t m32 = row >> 5;
   const int r = (int)(row & 31);
   const int units = c4n * 8;  // 16-k pieces of the row
@@ -100,10 +104,12 @@ __global__ __launch_bounds__(256) void k_af16split(
   };
   auto row_exponent = [&](float mx) {
     for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
-    __shared__ float wmx[4];
-    if ((t & 63) == 0) wmx[t >> 6] = mx;
-    __syncthreads();
-    mx = fmaxf(fmaxf(wmx[0], wmx[1]), fmaxf(wmx[2], wmx[3]));
+    if constexpr (TPR == 256) {
+      __shared__ float wmx[4];
+      if ((t & 63) == 0) wmx[t >> 6] = mx;
+      __syncthreads();
+      mx = fmaxf(fmaxf(wmx[0], wmx[1]), fmaxf(wmx[2], wmx[3]));
+    }
     int e = 0;
     if (mx > 0.f) {
       int ex;
@@ -1633,12 +1639,30 @@ NbitsPlan plan_nbits_ws(const mg_ctx *ctx, const mg_weight *w, int64_t M, int64_
       p.kwave = 1;
       ks = 1;
     }
-    // fp16 GEMM on at most three quarters of the CUs: up to three workgroups
-    // per CU from further K splits of at least 4 k groups, whose waits overlap
-    // (301 rows, 8192 -> 2048: 2 splits 66.0, 4 55.7, 8 52.3 us; 2048 -> 3072:
-    // 1 / 2 / 4 / 8 31.7 / 30.8 / 28.2 / 30.1; with 256 tiles none is faster).
-    if (p.path == 1 && wide && 4 * tiles <= 3 * target)
-      ks = std::max(ks, std::min(3 * target / tiles, d.c4 / 4));
+    // fp16 GEMM on at most three quarters of the CUs: further K splits, two to
+    // three workgroups per CU, whose waits overlap, where the sums are long enough
+    // to pay for the partials.  301 rows to 3072 columns (144 tiles), us a call at 1
+    // / 2 / 3 / 4 splits: K = 1024 19.5 / 21.6 / 22.6 / 23.6, 1536 26.0 / 27.0 / 25.5 /
+    // 26.8; of one split's time 2048 0.99 / 0.90 / 0.90, 8192 0.81 / 0.66 / 0.68; to 4096
+    // (192), K = 2048 0.99 / 0.97 / 0.92.  Of two's at 4 / 6 / 8: to 1536 (72), K = 3072
+    // 0.88 / 0.81 / 0.90; to 2048 (96), K = 4096 0.87 / 0.86 / 0.84; to 2560 (120) 0.89 /
+    // 0.94 / 0.95.  Of four's, 100 rows, K = 8192 at 8 / 16: to 2560 (40) 0.89 / 0.86, to
+    // 4096 (64) 0.93 / 1.02.  Many row tiles gain nothing (1500 rows to 768 columns, K =
+    // 4096: 60 / 66 / 69 / 66 us); the lines are at the last row tiles that do.
+    if (p.path == 1 && wide && 4 * tiles <= 3 * target) {
+      const int64_t c4 = d.c4;
+      if (2 * tiles > target) {
+        if (mt <= 8 && 3 * tiles <= 2 * target && c4 >= 12) ks = 3;
+        else if (mt <= 8 && c4 >= 16) ks = 4;
+      } else if (4 * tiles > target) {
+        if (mt <= 5 && c4 >= 16)
+          ks = 6 * tiles <= 2 * target ? 6 : c4 >= 32 && 8 * tiles <= 3 * target ? 8 : 4;
+      } else if (8 * tiles > target && mt <= 3) {
+        if (mt <= 2 && c4 >= 64 && 16 * tiles <= 3 * target) ks = 16;
+        else if (c4 >= 32) ks = 8;
+        else if (mt <= 2 && c4 >= 24 && 6 * tiles <= target) ks = 6;
+      }
+    }
     p.kps = (int)((d.c4 + ks - 1) / ks);
     p.ksplit = (int)((d.c4 + p.kps - 1) / p.kps);
     if (p.path == 4) {
@@ -2231,13 +2255,15 @@ mg_status prefill_run(mg_ctx *ctx, int n, const mg_weight *const *w, const float
   const int vec = (w0->K % 4 == 0) && (reinterpret_cast<uintptr_t>(a_dev) % 16 == 0);
   {
     const int pieces = (int)((d.c4 * 8 + 255) / 256);  // 16-k pieces per lane
-#define MG_SPLIT_LAUNCH(UL_)                                                                \
-  hipLaunchKernelGGL((k_af16split<UL_>), dim3((unsigned)p.mpad), dim3(256), 0, st, a_dev, M, \
-                     w0->K, (int)d.c4, vec, ahl, texp)
-    if (pieces == 1) MG_SPLIT_LAUNCH(1);
-    else if (pieces == 2) MG_SPLIT_LAUNCH(2);
-    else if (pieces <= 4) MG_SPLIT_LAUNCH(4);
-    else MG_SPLIT_LAUNCH(0);
+#define MG_SPLIT_LAUNCH(TPR_, UL_)                                                           \
+  hipLaunchKernelGGL((k_af16split<TPR_, UL_>), dim3((unsigned)(p.mpad * TPR_ / 256)), dim3(256), \
+                     0, st, a_dev, M, w0->K, (int)d.c4, vec, ahl, texp)
+    if (M >= 1024 && d.c4 <= 4) MG_SPLIT_LAUNCH(64, 1);
+    else if (p.mpad >= (int64_t)1 << 22) MG_SPLIT_LAUNCH(64, 0);
+    else if (pieces == 1) MG_SPLIT_LAUNCH(256, 1);
+    else if (pieces == 2) MG_SPLIT_LAUNCH(256, 2);
+    else if (pieces <= 4) MG_SPLIT_LAUNCH(256, 4);
+    else MG_SPLIT_LAUNCH(256, 0);
 #undef MG_SPLIT_LAUNCH
   }
   MG_TRY(mg_launch_check("k_af16split"));

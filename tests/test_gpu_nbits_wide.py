@@ -1,7 +1,7 @@
 """Prefill plans of the fp16 GEMM (blocks below 128): further K splits on grids
-of few tiles, 64-column tiles where wide ones would leave CUs without work, and
-the plan without them under a byte budget; against the oracle on a subset of
-columns."""
+of few tiles, 64-column tiles where wide ones would leave CUs without work, the
+forms of the activations' split, and the plan without further splits under a byte
+budget and under capture; against the oracle on a subset of columns."""
 import numpy as np
 import pytest
 
@@ -41,7 +41,15 @@ def check(y, a, w, k, bs):
     (129, 1024, 6145, 64),   # 194 tiles: above the line
     (301, 256, 16384, 32),   # 384 wide tiles: 768 narrow ones instead
     (256, 4128, 96, 32),     # few columns, 33 k groups
-])
+    (301, 1504, 3072, 32),   # 144 tiles, 12 k groups: 3 splits
+    (301, 1408, 3072, 32),   # 11: one
+    (140, 2016, 5500, 32),   # 172 tiles, 16 k groups: 4 splits
+    (300, 2080, 2100, 64),   # 99 tiles, 17 k groups: 4 splits, the last one short
+    (300, 4100, 2000, 32),   # 96 tiles, 33 k groups: 8 splits of 5 and fewer
+    (70, 4128, 2600, 32),    # 41 tiles: 8 splits for 4
+    (641, 4096, 1000, 32),   # 96 tiles in 6 rows of them: as without further splits
+    (1025, 200, 65, 32),     # activations split with a wave a row
+    (1023, 500, 65, 32), (1024, 512, 64, 32), (1024, 545, 64, 32)])
 def test_plans(ops, m, k, n, bs):
     rng = np.random.default_rng(m + k + n)
     w, h = weight(ops, rng, k, n, bs)
