@@ -37,7 +37,8 @@ struct ConvPair {
   int in_sp, out_sp, win_sp;
   int chunks, chunk;              // maxima chunks of an image, elements of each
   uint4 *wi, *xi;                 // images of the filters and of the input
-  int *we, *xe;                   // their words (pair_word; xe without the count)
+  int *we, *xe;                   // their words (pair_word) without the counts
+  int *wn;                        // small elements of filter m: four counts at 4 m
   int *xn;                        // small elements of image i at i * kCountStride
   unsigned *part;                 // [n][chunks] largest magnitudes (bits)
   int nx, pr, pc;                 // tile grid and its XCD cut
@@ -55,32 +56,26 @@ __global__ __launch_bounds__(256) void k_conv_pair_prep(const ConvPair p) {
   const float *src = filt ? p.w + (int64_t)m * K : p.x + img * xn + (int64_t)ch * p.chunk;
   const int len = filt ? (m < p.m ? K : 0)
                        : (int)std::min<int64_t>(p.chunk, xn - (int64_t)ch * p.chunk);
-  unsigned mx = 0, mn = ~0u;
+  unsigned mx = 0;
   for (int i = t; i < len; i += 8 * 256) {
     float v[8];
 #pragma unroll
     for (int u = 0; u < 8; u++) v[u] = src[min(i + 256 * u, len - 1)];
 #pragma unroll
-    for (int u = 0; u < 8; u++) {
-      mx = max(mx, __builtin_bit_cast(unsigned, v[u]) & 0x7fffffffu);
-      mn = min(mn, pair_bits1(v[u]));
-    }
+    for (int u = 0; u < 8; u++) mx = max(mx, __builtin_bit_cast(unsigned, v[u]) & 0x7fffffffu);
   }
-  for (int o = 32; o > 0; o >>= 1) {
-    mx = max(mx, (unsigned)__shfl_xor((int)mx, o));
-    mn = min(mn, (unsigned)__shfl_xor((int)mn, o));
-  }
-  __shared__ unsigned wmx[4], wmn[4];
-  if ((t & 63) == 0) wmx[t >> 6] = mx, wmn[t >> 6] = mn;
+  for (int o = 32; o > 0; o >>= 1) mx = max(mx, (unsigned)__shfl_xor((int)mx, o));
+  __shared__ unsigned wmx[4];
+  if ((t & 63) == 0) wmx[t >> 6] = mx;
   __syncthreads();
   mx = max(max(wmx[0], wmx[1]), max(wmx[2], wmx[3]));
-  mn = min(min(wmn[0], wmn[1]), min(wmn[2], wmn[3]));
   if (!filt) {
     if (t == 0) p.part[q] = mx;
     if (t == 0 && ch == 0) p.xn[img * kCountStride] = 0;
     return;
   }
   const int e = pair_exponent(mx);
+  if (t == 0) p.we[m] = pair_word(e, mx, 0);
   const unsigned below = pair_small_below(e);
   int small = 0;
   // Octet o: channels 8 c8 .. +7 of tap r, then the padding steps' zeros.
@@ -92,9 +87,8 @@ __global__ __launch_bounds__(256) void k_conv_pair_prep(const ConvPair p) {
 #pragma unroll
       for (int j = 0; j < 8; j++)
         if (8 * c8 + j < p.c) v[j] = src[(8 * c8 + j) * p.taps + r];
-    if (mn < below)  // uniform
 #pragma unroll
-      for (int j = 0; j < 8; j++) small += pair_bits1(v[j]) < below;
+    for (int j = 0; j < 8; j++) small += pair_bits1(v[j]) < below;
     half8 hi, lo;
     pair_split8(v, e, &hi, &lo);
     const int s = o < 2 * real ? (c8 >> 1) * p.taps + r : o >> 1, h = o < 2 * real ? c8 & 1 : o & 1;
@@ -102,14 +96,10 @@ __global__ __launch_bounds__(256) void k_conv_pair_prep(const ConvPair p) {
     d[0] = __builtin_bit_cast(uint4, hi);
     d[64] = __builtin_bit_cast(uint4, lo);
   }
-  if (mn < below) {
+  // A count of each wave: no barrier, and few have any to add up.
+  if (__ballot(small != 0))
     for (int o = 32; o > 0; o >>= 1) small += __shfl_xor(small, o);
-    __shared__ int wsm[4];
-    if ((t & 63) == 0) wsm[t >> 6] = small;
-    __syncthreads();
-    small = wsm[0] + wsm[1] + wsm[2] + wsm[3];
-  }
-  if (t == 0) p.we[m] = pair_word(e, mx, small);
+  if ((t & 63) == 0) p.wn[4 * m + (t >> 6)] = small;
 }
 
 // Thread = one position of the padded window, 16 channels (grid: positions,
@@ -231,7 +221,9 @@ __global__ __launch_bounds__(256, 2) void k_conv_pair(const ConvPair p) {
   }
   const int m0 = tr * 64, cols = p.n * p.out_sp, ns = p.ns, per = ns / 4;
   if (t < 64) {
-    exps[t] = p.we[m0 + t];
+    const int4 n = reinterpret_cast<const int4 *>(p.wn)[m0 + t];
+    const int w = p.we[m0 + t];
+    exps[t] = pair_word_small(w) ? w : w + (n.x + n.y + n.z + n.w) * 1024;
     const bool some = __ballot(pair_word_small(exps[t]) > 0) != 0;
     if (t == 0) count = some;
     bias[t] = p.bias && m0 + t < p.m ? p.bias[m0 + t] : 0.f;
@@ -308,7 +300,6 @@ __global__ __launch_bounds__(256, 2) void k_conv_pair(const ConvPair p) {
   // Without small elements in the tile's filters and images no output is redone.
   const bool check =  // uniform: every wave holds the tile's columns
       count != 0 || __ballot(pair_word_small(eb[0]) > 0 || pair_word_small(eb[1]) > 0) != 0;
-  const unsigned mask = check && mine ? pair_mask(part, wave, lane, wa, wj) : 0u;
   const __amdgpu_buffer_rsrc_t ry = rsrc(p.y);
   // The outputs in `which`; stores of the others go past the resource and are
   // dropped in hardware.
@@ -325,14 +316,15 @@ __global__ __launch_bounds__(256, 2) void k_conv_pair(const ConvPair p) {
           0, 0);
     }
   };
-  if (mine) {
-    float16v s;
+  float16v s;
 #pragma unroll
-    for (int v = 0; v < 16; v++)
-      s[v] = ldexpf(sum[v], -(pair_word_exp(wa[v]) + pair_word_exp(wj)));
-    finish(s, ~mask);
+  for (int v = 0; v < 16; v++) s[v] = ldexpf(sum[v], -(pair_word_exp(wa[v]) + pair_word_exp(wj)));
+  if (!check) {
+    if (mine) finish(s, ~0u);
+    return;
   }
-  if (!check) return;
+  const unsigned mask = mine ? pair_mask(part, wave, lane, wa, wj) : 0u;
+  if (mine) finish(s, ~mask);
   // (Copies: arrays indexed by a lambda's argument would be kept in LDS.)
   const int i0 = img[0], i1 = img[1], z0 = oz[0], z1 = oz[1], y0 = oy[0], y1 = oy[1], x0 = ox[0],
             x1 = ox[1];
@@ -343,14 +335,14 @@ __global__ __launch_bounds__(256, 2) void k_conv_pair(const ConvPair p) {
         return conv_f32_tile(p, m0 + 32 * (q >> 1), k ? i1 : i0, (k ? z1 : z0) - p.pad[0],
                              (k ? y1 : y0) - p.pad[1], (k ? x1 : x0) - p.pad[2], w, lane);
       },
-      [&](const float16v &s) __attribute__((always_inline)) { finish(s, mask); });
+      [&](const float16v &e) __attribute__((always_inline)) { finish(e, mask); });
 }
 
 struct Plan {
   bool ok = false;
   ConvPair q{};
   int64_t nb = 0;  // images per round of launches
-  size_t off_we = 0, off_xi = 0, off_xe = 0, off_xn = 0, off_part = 0, total = 0;
+  size_t off_we = 0, off_wn = 0, off_xi = 0, off_xe = 0, off_xn = 0, off_part = 0, total = 0;
 };
 
 Plan plan(const mg_conv_problem &p) {
@@ -382,9 +374,16 @@ Plan plan(const mg_conv_problem &p) {
   // products (they pass through memory three times here): [32, 256, 56] 1 x 1
   // to 64 channels 99 / 67, to 256 of [32, 1024, 14] 35 / 74; and channel
   // counts that the blocks of 16 more than double ([32, 3, 224] 7 x 7: 206 /
-  // 153).
-  if (p.c * taps < 256 || 16 * cb > 2 * p.c ||
-      (p.m * taps < 128 && p.n * p.c * in * 4 > (int64_t)8 << 20))
+  // 153).  And so do large inputs that a stride mostly skips, unless k_conv would
+  // have a long chain over k on few tiles (lines from 280 sizes of stride 2 to 4):
+  // 1 x 1 stride 3 to 256 channels of [32, 512, 56] 172 / 91, stride 2 of [1, 256,
+  // 112] 28 / 18.5; 4 x 4 stride 4 to 64 channels of [32, 512, 56] 497 / 393, but of
+  // [8, 512, 56] 0.31 of its time.
+  const int64_t mib = p.n * p.c * in * 4 >> 20;
+  const int64_t tiles = mp / 64 * ((p.n * out + 63) / 64);
+  if (p.c * taps < 256 || 16 * cb > 2 * p.c || (p.m * taps < 128 && mib >= 8) ||
+      (mib >= 8 && 30 * 256 * mib > p.c * taps * std::max<int64_t>(256, tiles)) ||
+      (mib >= 128 && p.m * taps * out < 128 * in))
     return r;
   // 32-bit offsets throughout, and the filter rows as laid out.
   if (p.w_ms != p.c * taps || p.w_cs != taps || p.c * taps > kPairMaxSmall || p.c * in >= lim ||
@@ -403,6 +402,8 @@ Plan plan(const mg_conv_problem &p) {
   size_t off = mg_align((size_t)(mp * ns * 64));
   r.off_we = off;
   off += mg_align((size_t)mp * 4);
+  r.off_wn = off;
+  off += (size_t)mp * 16;
   r.off_xi = off;
   off += mg_align((size_t)(r.nb * img));
   r.off_xe = off;
@@ -431,6 +432,7 @@ mg_status mg_conv_pair_run(mg_ctx *ctx, const mg_conv_problem &p, void *ws) {
   q.bias = static_cast<const float *>(p.bias);
   q.wi = reinterpret_cast<uint4 *>(base);
   q.we = reinterpret_cast<int *>(base + r.off_we);
+  q.wn = reinterpret_cast<int *>(base + r.off_wn);
   q.xi = reinterpret_cast<uint4 *>(base + r.off_xi);
   q.xe = reinterpret_cast<int *>(base + r.off_xe);
   q.xn = reinterpret_cast<int *>(base + r.off_xn);

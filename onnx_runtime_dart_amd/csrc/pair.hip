@@ -271,7 +271,6 @@ __global__ __launch_bounds__(256, 2) void k_pair_gemm(const PairArgs p) {
   // Without small elements in the tile's rows and columns no output is redone (a
   // barrier at the end of every workgroup took 3 us of FFN1's 32).
   const bool check = (counts[0] | counts[1]) != 0;  // uniform
-  const unsigned mask = check && mine ? pair_mask(part, wave, lane, wa, wb) : 0u;
   // y = alpha sum + beta C of the outputs in `which`.  Stores of the others, and
   // past M or N, go past the resource and are dropped in hardware.
   auto finish = [&](const float16v &s, unsigned which) __attribute__((always_inline)) {
@@ -299,21 +298,22 @@ __global__ __launch_bounds__(256, 2) void k_pair_gemm(const PairArgs p) {
                                             0, 0);
     }
   };
-  if (mine) {
-    float16v s;
+  float16v s;
 #pragma unroll
-    for (int v = 0; v < 16; v++)
-      s[v] = ldexpf(sum[v], -(pair_word_exp(wa[v]) + pair_word_exp(wb)));
-    finish(s, ~mask);
+  for (int v = 0; v < 16; v++) s[v] = ldexpf(sum[v], -(pair_word_exp(wa[v]) + pair_word_exp(wb)));
+  if (!check) {
+    if (mine) finish(s, ~0u);
+    return;
   }
-  if (!check) return;
+  const unsigned mask = mine ? pair_mask(part, wave, lane, wa, wb) : 0u;
+  if (mine) finish(s, ~mask);
   pair_redo(
       part, wave, lane, mask,
       [&](int q, int w) __attribute__((always_inline)) {
         return f32_tile(p.a, p.b, p.M, p.N, p.K, p.vec, r0 + 32 * (q >> 1), c0 + 32 * (q & 1), w,
                         lane);
       },
-      [&](const float16v &s) __attribute__((always_inline)) { finish(s, mask); });
+      [&](const float16v &e) __attribute__((always_inline)) { finish(e, mask); });
 }
 
 }  // namespace

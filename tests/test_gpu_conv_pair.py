@@ -103,6 +103,16 @@ def test_inf_and_nan(ops):
     np.testing.assert_array_equal(y[:, 65], np.sign(x[:, 0]) * np.float32(np.inf))
 
 
+@pytest.mark.parametrize("x,w,stride", [
+    ((8, 256, 33, 33), (40, 256, 1, 1), 3),    # 8.5 MiB, mostly skipped: on fp32 MFMA
+    ((3, 1030, 33, 25), (40, 1030, 1, 1), 3),  # 9.7 MiB, longer chain: on digit pairs
+    ((2, 256, 64, 65), (40, 256, 4, 4), 4)])
+def test_large_strided_inputs(ops, x, w, stride):
+    x, w, b = draw((x, w))
+    y = ops.op_conv(x, w, b, strides=[stride] * 2)
+    check(y, x, w, b, (stride,) * 2, (0,) * 4, (1, 1), redone=True)
+
+
 @pytest.mark.parametrize("big", [1e6, 1e12, 1e20, -3.4028235e38])
 @pytest.mark.parametrize("case", CASES[1:4] + CASES[7:], ids=lambda c: "x".join(map(str, c[0] + c[1])))
 def test_large_value_in_a_corner(ops, case, big):
