@@ -1646,21 +1646,23 @@ NbitsPlan plan_nbits_ws(const mg_ctx *ctx, const mg_weight *w, int64_t M, int64_
     // 26.8; of one split's time 2048 0.99 / 0.90 / 0.90, 8192 0.81 / 0.66 / 0.68; to 4096
     // (192), K = 2048 0.99 / 0.97 / 0.92.  Of two's at 4 / 6 / 8: to 1536 (72), K = 3072
     // 0.88 / 0.81 / 0.90; to 2048 (96), K = 4096 0.87 / 0.86 / 0.84; to 2560 (120) 0.89 /
-    // 0.94 / 0.95.  Of four's, 100 rows, K = 8192 at 8 / 16: to 2560 (40) 0.89 / 0.86, to
+    // 0.94 / 0.95; to 1488 (72), K = 1824, 26.0 us at 2, 23.6 at 3.  Of four's, 100 rows, K = 8192 at 8 / 16: to 2560 (40) 0.89 / 0.86, to
     // 4096 (64) 0.93 / 1.02.  Many row tiles gain nothing (1500 rows to 768 columns, K =
     // 4096: 60 / 66 / 69 / 66 us); the lines are at the last row tiles that do.
     if (p.path == 1 && wide && 4 * tiles <= 3 * target) {
       const int64_t c4 = d.c4;
       if (2 * tiles > target) {
-        if (mt <= 8 && 3 * tiles <= 2 * target && c4 >= 12) ks = 3;
+        if (mt <= 8 && 8 * tiles <= 5 * target && c4 >= 12) ks = 3;
         else if (mt <= 8 && c4 >= 16) ks = 4;
       } else if (4 * tiles > target) {
         if (mt <= 5 && c4 >= 16)
           ks = 6 * tiles <= 2 * target ? 6 : c4 >= 32 && 8 * tiles <= 3 * target ? 8 : 4;
+        else if (mt <= 5 && c4 >= 12 && 3 * tiles <= target)
+          ks = 3;
       } else if (8 * tiles > target && mt <= 3) {
         if (mt <= 2 && c4 >= 64 && 16 * tiles <= 3 * target) ks = 16;
         else if (c4 >= 32) ks = 8;
-        else if (mt <= 2 && c4 >= 24 && 6 * tiles <= target) ks = 6;
+        else if (mt <= 2 && c4 >= 24 && 16 * 6 * tiles <= 17 * target) ks = 6;
       }
     }
     p.kps = (int)((d.c4 + ks - 1) / ks);
