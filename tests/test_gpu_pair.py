@@ -192,6 +192,28 @@ def test_ranges_within_a_row(ops, k, off):
     ad.free()
 
 
+@pytest.mark.parametrize("c_shape", [(1,), (130,), (70, 1), (70, 130)])
+def test_redone_outputs_with_c(ops, c_shape):
+    # alpha and beta C on outputs of both forms in one tile, C also in place.
+    rng = np.random.default_rng(11)
+    m, k, n = 70, 320, 130
+    s = rng.integers(-40, 41, k)
+    a = (rng.standard_normal((m, k)) * 2.0**s).astype(np.float32)
+    w = (rng.standard_normal((n, k)) * 2.0**-s).astype(np.float32)
+    a[::3], w[::2] = rng.standard_normal((24, k)), rng.standard_normal((65, k))
+    a[::6, 9], w[:, 9] = 1e30, 0
+    c = rng.standard_normal(c_shape).astype(np.float32)
+    fw = ops.F32Weight(w, trans_b=True)
+    check(fw.gemm(a, c, alpha=0.5, beta=2.0), a, w, c, 0.5, 2.0)
+    if c.shape == (m, n):
+        ad, yd = ops.DeviceBuffer.from_array(a), ops.DeviceBuffer.from_array(c)
+        fw.gemm_dev(ad.ptr, m, yd.ptr, yd.ptr, c.shape, alpha=0.5, beta=2.0)
+        check(yd.to_array((m, n), np.float32), a, w, c, 0.5, 2.0)
+        ad.free()
+        yd.free()
+    fw.release()
+
+
 def test_inf_and_nan_beside_small(ops):
     # As test_inf_and_nan, at a K of the pairs, with rows of zeros and of small
     # elements among them: 0 Inf is NaN, as the sum in fp32 gives it.
