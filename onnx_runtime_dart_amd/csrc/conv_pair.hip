@@ -42,6 +42,7 @@ struct ConvPair {
   int *xn;                        // small elements of image i at i * kCountStride
   unsigned *part;                 // [n][chunks] largest magnitudes (bits)
   int nx, pr, pc;                 // tile grid and its XCD cut
+  int wvec;                       // the filters' rows are 16-byte aligned
 };
 
 // Bound by latency (a few loads per thread, one round trip each way): the
@@ -148,29 +149,51 @@ __global__ __launch_bounds__(256) void k_conv_pair_x(const ConvPair p) {
 
 // One wave's quarter of the sums of the 32 x 32 block of channels m0 .. and
 // columns of which lane l's is (img, window origin oz, oy, ox), on fp32 MFMA
-// straight from the tensors: steps of 16 channels at one tap, MFMA i of a step
-// channel 2 i for lanes 0-31 and 2 i + 1 for 32-63, the next step's loads in
-// flight.  Channels past m repeat the last one; nobody stores their sums.
+// straight from the tensors.  Lanes 0-31 take the first half of the quarter's k =
+// (channel, tap) and 32-63 the second, each in order, so that eight k of a filter
+// are two 16-byte loads (wvec: rows are aligned for it) and the tap advances by
+// counting; the next eight are on their way during the products.  Channels past m
+// repeat the last one; nobody stores their sums.  ResNet-50's 3 x 3 takes 202 us
+// where one of its 32 images has a NaN and 248 where each has (steps of 16 channels
+// at one tap, whose filter loads touch a line per lane: 200 / 346; the same with the
+// tap advanced by selects in place of branches: 230 / 306).
 __device__ inline float16v conv_f32_tile(const ConvPair &p, int m0, int img, int oz, int oy, int ox,
                                          int wave, int lane) {
-  const int h = lane >> 5, real = p.cb * p.taps, per = (real + 3) / 4;
-  const int s0 = wave * per, s1 = min(real, s0 + per);
-  const float *w = p.w + (int64_t)min(m0 + (lane & 31), p.m - 1) * p.c * p.taps;
+  const int K = p.c * p.taps, half = (K + 63) / 64 * 8, steps = half / 8;
+  int k = (2 * wave + (lane >> 5)) * half;  // of the next load
+  const float *w = p.w + (int64_t)min(m0 + (lane & 31), p.m - 1) * K;
   const float *x = p.x + (int64_t)img * p.c * p.in_sp;
+  const int ch = k / p.taps, tap = k - ch * p.taps;
+  int kx = tap % p.ker[2], ky = tap / p.ker[2] % p.ker[1], kz = tap / p.ker[2] / p.ker[1];
+  int ix = ox + kx * p.dil[2], iy = oy + ky * p.dil[1], iz = oz + kz * p.dil[0];
+  int64_t xc = (int64_t)ch * p.in_sp;
   float a[2][8], b[2][8];
-  auto load = [&](int d, int s) __attribute__((always_inline)) {
-    const int c0 = s / p.taps * 16, tap = s % p.taps;
-    const int kx = tap % p.ker[2], ky = tap / p.ker[2] % p.ker[1], kz = tap / p.ker[2] / p.ker[1];
-    const int iz = oz + kz * p.dil[0], iy = oy + ky * p.dil[1], ix = ox + kx * p.dil[2];
-    const bool ok = (unsigned)iz < (unsigned)p.in[0] && (unsigned)iy < (unsigned)p.in[1] &&
-                    (unsigned)ix < (unsigned)p.in[2];
-    const float *xt = x + (ok ? (iz * p.in[1] + iy) * p.in[2] + ix : 0);
+  auto load = [&](int d) __attribute__((always_inline)) {
+    if (p.wvec) {
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-      const int ch = c0 + 2 * j + h, cc = min(ch, p.c - 1);
-      const float av = w[cc * p.taps + tap], bv = xt[(int64_t)cc * p.in_sp];
-      a[d][j] = ch < p.c ? av : 0.f;
-      b[d][j] = ch < p.c && ok ? bv : 0.f;
+      for (int q = 0; q < 2; q++) {
+        const float4v v =
+            k + 4 * q < K ? *reinterpret_cast<const float4v *>(w + k + 4 * q) : (float4v){};
+#pragma unroll
+        for (int i = 0; i < 4; i++) a[d][4 * q + i] = v[i];
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; j++) a[d][j] = k + j < K ? w[k + j] : 0.f;
+    }
+#pragma unroll
+    for (int j = 0; j < 8; j++, k++) {
+      const bool ok = k < K && (unsigned)iz < (unsigned)p.in[0] &&
+                      (unsigned)iy < (unsigned)p.in[1] && (unsigned)ix < (unsigned)p.in[2];
+      b[d][j] = ok ? x[xc + (iz * p.in[1] + iy) * p.in[2] + ix] : 0.f;
+      ix += p.dil[2];
+      if (++kx == p.ker[2]) {
+        kx = 0, ix = ox, iy += p.dil[1];
+        if (++ky == p.ker[1]) {
+          ky = 0, iy = oy, iz += p.dil[0];
+          if (++kz == p.ker[0]) kz = 0, iz = oz, xc += p.in_sp;
+        }
+      }
     }
   };
   float16v acc = {};
@@ -179,13 +202,13 @@ __device__ inline float16v conv_f32_tile(const ConvPair &p, int m0, int img, int
     for (int j = 0; j < 8; j++)
       acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[d][j], b[d][j], acc, 0, 0, 0);
   };
-  if (s0 >= s1) return acc;
-  load(0, s0);
-  for (int s = s0; s < s1; s += 2) {
-    load(1, min(s + 1, s1 - 1));
+  load(0);
+  for (int s = 0; s < steps; s += 2) {
+    if (s + 1 < steps) load(1);
     step(0);
-    load(0, min(s + 2, s1 - 1));
-    if (s + 1 < s1) step(1);
+    if (s + 1 == steps) break;
+    if (s + 2 < steps) load(0);
+    step(1);
   }
   return acc;
 }
@@ -437,6 +460,7 @@ mg_status mg_conv_pair_run(mg_ctx *ctx, const mg_conv_problem &p, void *ws) {
   q.xe = reinterpret_cast<int *>(base + r.off_xe);
   q.xn = reinterpret_cast<int *>(base + r.off_xn);
   q.part = reinterpret_cast<unsigned *>(base + r.off_part);
+  q.wvec = q.c * q.taps % 4 == 0 && reinterpret_cast<uintptr_t>(p.w) % 16 == 0;
   const int mp = (q.m + 63) / 64 * 64;
   for (int64_t n0 = 0; n0 < p.n; n0 += r.nb) {
     q.n = (int)std::min(r.nb, p.n - n0);
